@@ -151,6 +151,18 @@ int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
 int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                     const afd_ws_layout& L, int32_t n, hipStream_t stream);
 
+// Grouped GEMMs for few tokens per expert (afd_gemm_rows.hip), every format; the same results bit
+// for bit. few_rows: whether a call of n tokens takes them.
+constexpr int kFewRowsPerExpert = 40;
+bool few_rows(const afd_moe_cfg& cfg, int32_t n);
+// x / xs: the token rows in the activation format (quantized, or bf16 with xs null); with
+// rows_desc != nullptr they are read from that job descriptor when the kernel runs.
+int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
+                        const afd_ws_layout& L, const void* x, const void* xs,
+                        const afd_job* rows_desc, int32_t n, hipStream_t stream);
+int launch_rows_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
+                     const afd_ws_layout& L, int32_t n, hipStream_t stream);
+
 // Number of compute units of the current device (cached per device).
 int device_cu_count();
 

@@ -1,0 +1,90 @@
+"""GPU: the few-rows GEMMs (calls with few tokens per expert), every weight and activation
+format, at the sizes where they can go wrong: expert counts around the 32-row blocks, the
+64-row groups and the row tiles (128, or 256 for FP8 block weights with fp8 activations), experts
+with no row, one K stage and K stages that do not fill the register ring, one and several weight
+image columns, and an expert count that is not a multiple of the 4 a lane looks up.
+
+The large-tile GEMMs and the few-rows GEMMs feed every accumulator the same products in the
+same order, so the same tokens inside a call large enough for the large tiles must give the
+same bits; against the oracle the bar is that of the other layer tests (rel-L2 1e-2: the same
+quantizers at the same points, another order of the fp32 sums)."""
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import bits16, dev, rel_l2, say
+from oracle import experts as OX
+from oracle import formats as F
+from sgl_asap_amd import workloads as W
+from sgl_asap_amd.moe.experts import AfdExperts, pack_fp8_block_experts, pack_mxfp4_experts
+from sgl_asap_amd.moe.topk import StandardTopKOutput
+from test_gpu_moe import deq_weights
+
+pytestmark = pytest.mark.gpu
+
+REL_L2_TOL = 1e-2
+# rows of the first experts; the others get none
+COUNTS = [1, 0, 31, 32, 33, 63, 64, 65, 127, 128, 129, 0, 2, 255, 256, 257, 7]
+# tokens per local expert up to which a call takes the few-rows GEMMs (topk 1 here)
+FEW_ROWS = 40
+
+
+def ids_for(counts, num_local, total, gen):
+    """total tokens, top-1: counts[e] of them on expert e, the others on no local expert, in
+    random order."""
+    ids = torch.full((total,), num_local, dtype=torch.int32)
+    at = 0
+    for e, c in enumerate(counts):
+        ids[at:at + c] = e
+        at += c
+    return ids[torch.randperm(total, generator=gen)][:, None].contiguous()
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block"])
+@pytest.mark.parametrize(
+    "hidden,inter,activation",
+    [
+        (256, 128, "silu"),  # 2 and 1 K stages, one image column in each GEMM
+        (768, 384, "silu_limit"),  # 6 and 3 K stages, 3 columns
+        (1280, 1152, "situ"),  # 10 and 9 K stages
+    ],
+)
+def test_few_rows_match_large_tiles(hidden, inter, activation, fmt, act):
+    num_local = 42
+    n, more = sum(COUNTS) + 5, FEW_ROWS * num_local + 1
+    assert n <= FEW_ROWS * num_local
+    say(f"few rows H={hidden} I={inter} {activation} {fmt} {act} n={n}")
+    gen = W.generator("cpu", 17)
+    x = W.tokens(n + more, hidden, gen, "cpu")
+    w = torch.rand(n + more, 1, generator=gen) + 0.25
+    ids = torch.cat([ids_for(COUNTS, num_local, n, gen),
+                     torch.randint(0, num_local + 1, (more, 1), generator=gen, dtype=torch.int32)])
+    w13, w2 = W.expert_weights(num_local, hidden, inter, gen, "cpu")
+    pack = pack_mxfp4_experts if fmt == "mxfp4" else pack_fp8_block_experts
+    kw, oact = {}, {}
+    if activation == "situ":
+        kw = dict(activation="situ", gemm1_alpha=2.0, gemm1_clamp_limit=3.0)
+        oact = dict(activation="situ", act_alpha=2.0, act_limit=3.0)
+    elif activation == "silu_limit":
+        kw, oact = dict(swiglu_limit=0.5), dict(activation="swiglu_limit", act_limit=0.5)
+    experts = AfdExperts(num_local + 1, 1, 0, range(num_local), pack(w13, w2, device=dev()), n_max=n + more,
+                         act_format="bf16" if act == "bf16" else None, **kw)
+
+    def call(m):
+        out = experts(x[:m].to(dev()), StandardTopKOutput(w[:m].to(dev()), ids[:m].to(dev())))
+        torch.cuda.synchronize()
+        return bits16(out)
+
+    few = call(n)
+    assert np.array_equal(few, call(n + more)[:n])
+    quant = "bf16" if act == "bf16" else "mxfp8" if fmt == "mxfp4" else "fp8_1x128"
+    ref = OX.moe_ffn(x[:n], ids[:n].numpy(), w[:n].numpy(), *deq_weights(w13, w2, fmt), 0, act=quant, **oact)
+    err = rel_l2(F.bf16_to_f32(few), F.bf16_to_f32(ref))
+    say(f"rel_l2={err:.3e}")
+    assert err <= REL_L2_TOL, err
+    # one token on one expert, alone and on the last expert
+    for e in (0, num_local - 1):
+        ids[:1] = e
+        assert np.array_equal(call(1), call(n + more)[:1]), e
