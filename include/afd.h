@@ -355,7 +355,8 @@ int afd_quant_act(const afd_moe_cfg* cfg, const uint16_t* x, int32_t n, uint8_t*
 
 /* afd_moe_ffn with hipEvent_t handles recorded on `stream` around its stages:
  * stage_events[0] before routing, [1] after the launch that histograms the pairs and
- * quantizes the activations, [2] after the router's scan and scatter, [3] after gate_up,
+ * quantizes the activations, [2] after the router's scan and scatter (with at most 4096 pairs
+ * both are one launch, and [1] and [2] both follow it), [3] after gate_up,
  * [4] after down, [5] after finalize. NULL entries are skipped.
  * Same replaced interface as afd_moe_ffn; for the per-stage timing of JobTimer
  * (P/srt/managers/scheduler.py:109-159). */

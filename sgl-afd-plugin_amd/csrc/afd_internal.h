@@ -120,7 +120,7 @@ int launch_quant_act(const afd_moe_cfg& cfg, const uint16_t* x, int32_t n, uint8
 // Routing of the job's pairs into the workspace; with quantize, the activation quantization
 // of job.x into ws.xq / ws.xs (MXFP8 in stage order, or FP8 1x128, by cfg.weight_fmt) runs
 // beside the expert histogram (without, the rows are quantized already). `mid` (optional)
-// is recorded between the two launches.
+// is recorded between the two launches (with few pairs there is one, and it follows that).
 // The first launch also zeroes the call's counter words.
 int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, uint8_t* ws,
                        const afd_ws_layout& L, hipStream_t stream, hipEvent_t mid);

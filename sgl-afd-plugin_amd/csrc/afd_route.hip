@@ -1,6 +1,9 @@
 // Routing of one job's (token, k) pairs to this F rank's local experts, on gfx950.
 //
-// Two launches, integer work on a 4*n*k-byte id array (HBM/latency bound):
+// Integer work on a 4*n*k-byte id array (HBM/latency bound). Two launches, or with few pairs one
+// (each workgroup of the second then counts the pairs by itself, at most 16 loads a thread, which
+// overlap, while workgroups beside it quantize; 15 -> 10 us of routing for 24 tokens of 64 FP8
+// experts):
 //   1. route_prep:    workgroup c < chunks histograms chunk c of the flat pair array by local
 //                     expert (LDS atomics; counts are order-free); with the expert call, the
 //                     remaining workgroups quantize the activations meanwhile (afd_quant_dev.h).
@@ -9,8 +12,8 @@
 //                     16-byte loads issued together) to get each expert's count, its own chunk's
 //                     base per expert and the block_m-padded expert offsets (a wavefront scan);
 //                     workgroup 0 also writes
-//                     counts, offsets, padded offsets, the row-tile table, the tile count and
-//                     the -1 fill of padding rows. It then walks its pairs in flat order, 256 at
+//                     counts, offsets, padded offsets, the row-tile table and the tile count;
+//                     the -1 fill of padding rows is dealt to all workgroups. It then walks its pairs in flat order, 256 at
 //                     a time; a pair's rank among equal keys inside its wavefront comes from 9
 //                     ballots (one per key bit), across wavefronts from LDS counts, so the
 //                     placement is the stable order (ascending flat index inside each expert)
@@ -23,6 +26,8 @@ namespace afd {
 
 constexpr int kRouteThreads = 256;
 constexpr int kMaxChunks = 128;
+constexpr int kFusedPairs = 4096;  // up to as many pairs are routed in one launch
+constexpr int kFusedGroups = 16;   // by at least as many workgroups (they share the -1 fill)
 constexpr int kKeyBits = 9;  // keys 0..256 (local expert, or num_local for "not local")
 static_assert(kRouteThreads == kQuantThreads, "the prep kernel's workgroups do either job");
 
@@ -39,26 +44,37 @@ struct PrepQuant {
   void* s;
 };
 
+// workgroup b of g quantizes its share of the job's rows
+template <int QUANT>
+__device__ __forceinline__ void quant_share(const JobIn& job, const PrepQuant& pq, int b, int g) {
+  const int64_t first = int64_t(b) * kRouteThreads + threadIdx.x;
+  const int64_t stride = int64_t(g) * kRouteThreads;
+  const int64_t items = job.n * (pq.cols / kMxBlock);
+  const int cols = pq.cols;
+  auto xrow = [&job, cols](int64_t r) { return job_x_row(job, r, cols); };
+  if constexpr (QUANT == kPrepMxfp8)
+    quant_mxfp8_items<true>(xrow, items, cols, pq.q, static_cast<uint8_t*>(pq.s), first, stride);
+  else if constexpr (QUANT == kPrepFp8)
+    quant_fp8_1x128_items(xrow, items, cols, pq.q, static_cast<float*>(pq.s), first, stride);
+}
+
+// zeroes the call's counter words (one wavefront)
+__device__ __forceinline__ void zero_counters(uint32_t* counters) {
+  if (threadIdx.x < kCounterLines) {
+    uint32_t* line = counters + kLineWord0 + threadIdx.x * kLineStride;
+    line[0] = line[1] = line[2] = 0u;
+    if (threadIdx.x == 0) counters[kArriveWord] = 0u;
+  }
+}
+
 template <int QUANT>
 __global__ __launch_bounds__(kRouteThreads) void route_prep_kernel(
     JobIn jin, int topk, int chunk, int chunks, int e_lo, int num_local,
     int32_t* __restrict__ hist, PrepQuant pq, uint32_t* __restrict__ counters) {
   const JobIn job = resolve_job(jin);
-  if (blockIdx.x == 0 && threadIdx.x < kCounterLines) {
-    uint32_t* line = counters + kLineWord0 + threadIdx.x * kLineStride;
-    line[0] = line[1] = line[2] = 0u;
-    if (threadIdx.x == 0) counters[kArriveWord] = 0u;
-  }
+  if (blockIdx.x == 0) zero_counters(counters);
   if (static_cast<int>(blockIdx.x) >= chunks) {
-    const int64_t first = (int64_t(blockIdx.x) - chunks) * kRouteThreads + threadIdx.x;
-    const int64_t stride = (int64_t(gridDim.x) - chunks) * kRouteThreads;
-    const int64_t items = job.n * (pq.cols / kMxBlock);
-    const int cols = pq.cols;
-    auto xrow = [&job, cols](int64_t r) { return job_x_row(job, r, cols); };
-    if constexpr (QUANT == kPrepMxfp8)
-      quant_mxfp8_items<true>(xrow, items, cols, pq.q, static_cast<uint8_t*>(pq.s), first, stride);
-    else if constexpr (QUANT == kPrepFp8)
-      quant_fp8_1x128_items(xrow, items, cols, pq.q, static_cast<float*>(pq.s), first, stride);
+    quant_share<QUANT>(job, pq, blockIdx.x - chunks, gridDim.x - chunks);
     return;
   }
   const int64_t pairs = job.n * topk;
@@ -76,13 +92,23 @@ __global__ __launch_bounds__(kRouteThreads) void route_prep_kernel(
     hist[int64_t(e) * kMaxChunks + blockIdx.x] = cnt[e];
 }
 
+// kFused (few pairs): the first `route_groups` workgroups count the pairs themselves instead of
+// reading a histogram, and the others quantize, so there is no launch before this one.
+template <bool kFused, int QUANT>
 __global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
-    JobIn jin, int topk, int chunk, int chunks, int e_lo, int num_local, int block_m,
+    JobIn jin, int topk, int chunk, int chunks, int route_groups, int e_lo, int num_local, int block_m,
     const int32_t* __restrict__ hist, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ poff, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tile_expert,
-    int32_t* __restrict__ num_tiles) {
+    int32_t* __restrict__ num_tiles, PrepQuant pq, uint32_t* __restrict__ counters) {
   const JobIn job = resolve_job(jin);
+  if constexpr (kFused) {
+    if (blockIdx.x == 0) zero_counters(counters);
+    if (static_cast<int>(blockIdx.x) >= route_groups) {
+      quant_share<QUANT>(job, pq, blockIdx.x - route_groups, gridDim.x - route_groups);
+      return;
+    }
+  }
   const int64_t pairs = job.n * topk;
   constexpr int kWaves = kRouteThreads / 64;
   __shared__ int run[kMaxLocalExperts + 1];
@@ -98,39 +124,53 @@ __global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
   // histogram pass; each later batch is loaded two batches ahead
   int id_cur = lo + t < hi ? job_id(job, lo + t, topk) : 0;
   int id_nxt = lo + kRouteThreads + t < hi ? job_id(job, lo + kRouteThreads + t, topk) : 0;
-  // Expert e's chunks are split over G = kRouteThreads / num_local threads (e, g), each summing
-  // a contiguous run of them (a multiple of 4 long, so 16-byte loads of the expert's row of the
-  // histogram; entries at or past `chunks` are never written and are masked): the counts in
-  // all chunks and in the chunks before this one.
   const int G = kRouteThreads / num_local;
-  const int per = ((chunks + G - 1) / G + 3) & ~3;
   const int e = t % num_local, g = t / num_local;
   const bool active = g < G;
-  const int c0 = active ? g * per : 0, c1 = active ? min(c0 + per, chunks) : 0;
-  int all = 0, before = 0;
-  const int32_t* hrow = hist + int64_t(e) * kMaxChunks;
-#pragma unroll 8
-  for (int k4 = c0; k4 < c1; k4 += 4) {
-    const v4i h = *reinterpret_cast<const v4i*>(hrow + k4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int v = k4 + j < c1 ? h[j] : 0;
-      all += v;
-      before += k4 + j < c ? v : 0;
-    }
-  }
-  part_all[t] = all;
-  part_before[t] = before;
   for (int i = t; i < kWaves * (kMaxLocalExperts + 1); i += kRouteThreads) (&wcnt[0][0])[i] = 0;
-  __syncthreads();
-  if (active && g == 0) {
-    int a = 0, b = 0;
-    for (int h = 0; h < G; ++h) {
-      a += part_all[h * num_local + e];
-      b += part_before[h * num_local + e];
+  if constexpr (kFused) {
+    // the counts of all pairs and of those before this chunk (LDS atomics; counts are order-free)
+    for (int i = t; i < num_local; i += kRouteThreads) tot[i] = run[i] = 0;
+    __syncthreads();
+#pragma unroll 4
+    for (int64_t i = t; i < pairs; i += kRouteThreads) {
+      const int key = pair_key(job_id(job, i, topk), e_lo, num_local);
+      if (key < num_local) {
+        atomicAdd(&tot[key], 1);
+        if (i < lo) atomicAdd(&run[key], 1);
+      }
     }
-    tot[e] = a;
-    run[e] = b;  // this chunk's rank base inside expert e; the segment start is added below
+  } else {
+    // Expert e's chunks are split over G = kRouteThreads / num_local threads (e, g), each summing
+    // a contiguous run of them (a multiple of 4 long, so 16-byte loads of the expert's row of the
+    // histogram; entries at or past `chunks` are never written and are masked): the counts in
+    // all chunks and in the chunks before this one.
+    const int per = ((chunks + G - 1) / G + 3) & ~3;
+    const int c0 = active ? g * per : 0, c1 = active ? min(c0 + per, chunks) : 0;
+    int all = 0, before = 0;
+    const int32_t* hrow = hist + int64_t(e) * kMaxChunks;
+#pragma unroll 8
+    for (int k4 = c0; k4 < c1; k4 += 4) {
+      const v4i h = *reinterpret_cast<const v4i*>(hrow + k4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int v = k4 + j < c1 ? h[j] : 0;
+        all += v;
+        before += k4 + j < c ? v : 0;
+      }
+    }
+    part_all[t] = all;
+    part_before[t] = before;
+    __syncthreads();
+    if (active && g == 0) {
+      int a = 0, b = 0;
+      for (int h = 0; h < G; ++h) {
+        a += part_all[h * num_local + e];
+        b += part_before[h * num_local + e];
+      }
+      tot[e] = a;
+      run[e] = b;  // this chunk's rank base inside expert e; the segment start is added below
+    }
   }
   __syncthreads();
   // expert offsets and block_m-padded offsets: one wavefront, 4 experts per lane
@@ -178,14 +218,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
   }
   __syncthreads();
   for (int ex = t; ex < num_local; ex += kRouteThreads) run[ex] += pof[ex];
-  if (c == 0) {
-    // row-tile table (thread e writes expert e's tiles) and -1 on the padding rows of every
-    // segment (the G threads of expert e stride over its at most block_m - 1 padding rows)
-    if (t < num_local)
-      for (int i = pof[t] / block_m, i1 = pof[t + 1] / block_m; i < i1; ++i) tile_expert[i] = t;
-    if (active)
-      for (int r = pof[e] + tot[e] + g; r < pof[e + 1]; r += G) sorted_pairs[r] = -1;
-  }
+  // row-tile table (thread e writes expert e's tiles) and -1 on the at most block_m - 1 padding
+  // rows of every segment, the experts dealt to all workgroups (by one workgroup the 16000
+  // padding rows of 64 small FP8 segments took 5 us)
+  if (c == 0 && t < num_local)
+    for (int i = pof[t] / block_m, i1 = pof[t + 1] / block_m; i < i1; ++i) tile_expert[i] = t;
+  const int groups = kFused ? route_groups : gridDim.x;
+  for (int ex = c; ex < num_local; ex += groups)
+    for (int r = pof[ex] + tot[ex] + t; r < pof[ex + 1]; r += kRouteThreads) sorted_pairs[r] = -1;
   __syncthreads();
   const uint64_t below = (uint64_t(1) << lane) - 1;
   for (int64_t base = lo; base < hi; base += kRouteThreads) {
@@ -249,33 +289,42 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
   PrepQuant pq{cfg.hidden, ws + L.xq, ws + L.xs};
   int quant_grid = 0;
   const int fmt = !quantize ? kPrepNone : cfg.weight_fmt == AFD_W_MXFP4 ? kPrepMxfp8 : kPrepFp8;
-  if (fmt != kPrepNone) quant_grid = grid_for(job.n * (cfg.hidden / kMxBlock));
-  if (job.n > 0 && chunks + quant_grid > 0) {
-    const dim3 grid(chunks + quant_grid);
-    if (fmt == kPrepMxfp8)
-      hipLaunchKernelGGL(route_prep_kernel<kPrepMxfp8>, grid, dim3(kRouteThreads), 0, stream, job,
-                         cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
-    else if (fmt == kPrepFp8)
-      hipLaunchKernelGGL(route_prep_kernel<kPrepFp8>, grid, dim3(kRouteThreads), 0, stream, job,
-                         cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
-    else
-      hipLaunchKernelGGL(route_prep_kernel<kPrepNone>, grid, dim3(kRouteThreads), 0, stream, job,
-                         cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
+  if (fmt != kPrepNone && job.n > 0) quant_grid = grid_for(job.n * (cfg.hidden / kMxBlock));
+  // at least one routing workgroup, which writes the (empty) tables when there are no pairs
+  auto scatter = [&](auto kernel, int route_groups, int grid) -> int {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kRouteThreads), 0, stream, job, cfg.topk, chunk, chunks,
+                       route_groups, cfg.expert_lo, cfg.num_local, L.block_m, hist,
+                       reinterpret_cast<int32_t*>(ws + L.counts), reinterpret_cast<int32_t*>(ws + L.offsets),
+                       reinterpret_cast<int32_t*>(ws + L.padded_offsets),
+                       reinterpret_cast<int32_t*>(ws + L.sorted_pairs),
+                       reinterpret_cast<int32_t*>(ws + L.pair_pos),
+                       reinterpret_cast<int32_t*>(ws + L.tile_expert),
+                       reinterpret_cast<int32_t*>(ws + L.num_tiles), pq, counters);
     AFD_CHECK_LAUNCH();
+    return AFD_OK;
+  };
+  if (pairs <= kFusedPairs) {
+    const int route_groups = chunks > kFusedGroups ? chunks : kFusedGroups;
+    const int grid = route_groups + quant_grid;
+    const int st = fmt == kPrepMxfp8 ? scatter(route_scatter_kernel<true, kPrepMxfp8>, route_groups, grid)
+                   : fmt == kPrepFp8 ? scatter(route_scatter_kernel<true, kPrepFp8>, route_groups, grid)
+                                     : scatter(route_scatter_kernel<true, kPrepNone>, route_groups, grid);
+    if (st == AFD_OK && mid) AFD_CHECK_HIP(hipEventRecord(mid, stream));
+    return st;
   }
-  if (mid) AFD_CHECK_HIP(hipEventRecord(mid, stream));
-  // at least one workgroup, which writes the (empty) tables when there are no pairs
-  hipLaunchKernelGGL(route_scatter_kernel, dim3(chunks > 0 ? chunks : 1), dim3(kRouteThreads), 0,
-                     stream, job, cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local,
-                     L.block_m, hist, reinterpret_cast<int32_t*>(ws + L.counts),
-                     reinterpret_cast<int32_t*>(ws + L.offsets),
-                     reinterpret_cast<int32_t*>(ws + L.padded_offsets),
-                     reinterpret_cast<int32_t*>(ws + L.sorted_pairs),
-                     reinterpret_cast<int32_t*>(ws + L.pair_pos),
-                     reinterpret_cast<int32_t*>(ws + L.tile_expert),
-                     reinterpret_cast<int32_t*>(ws + L.num_tiles));
+  const dim3 grid(chunks + quant_grid);
+  if (fmt == kPrepMxfp8)
+    hipLaunchKernelGGL(route_prep_kernel<kPrepMxfp8>, grid, dim3(kRouteThreads), 0, stream, job,
+                       cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
+  else if (fmt == kPrepFp8)
+    hipLaunchKernelGGL(route_prep_kernel<kPrepFp8>, grid, dim3(kRouteThreads), 0, stream, job,
+                       cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
+  else
+    hipLaunchKernelGGL(route_prep_kernel<kPrepNone>, grid, dim3(kRouteThreads), 0, stream, job,
+                       cfg.topk, chunk, chunks, cfg.expert_lo, cfg.num_local, hist, pq, counters);
   AFD_CHECK_LAUNCH();
-  return AFD_OK;
+  if (mid) AFD_CHECK_HIP(hipEventRecord(mid, stream));
+  return scatter(route_scatter_kernel<false, kPrepNone>, chunks, chunks);
 }
 
 }  // namespace afd
