@@ -74,6 +74,7 @@ struct A16GemmArgs {
   uint8_t* h_img;  // gate_up out: the down GEMM's bf16 A images [row tiles][N/2 / stage K]
   ActParams act;   // gate_up: the activation
   uint16_t* y;     // down out: bf16 [np][N]
+  RowsGate gate;   // whether this launch or the few-rows GEMM runs
 };
 
 // byte offset of logical 16-byte chunk c (0..15, 8 bf16 each) of row r in an A16 image: the
@@ -166,6 +167,8 @@ __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A
   using T = A16Tile<WF, WN>;
   using F = typename T::F;
   constexpr bool kFp8 = WF == kWFp8;
+  if constexpr (!kFp8)  // FP8 weights: never gated
+    if (p.gate.large_skips()) return;
   constexpr int kBM = T::kBM, kBN = T::kBN, kStages = T::kStages, kStage = T::kStage;
   constexpr int kStageK = T::kStageK, kPhases = T::kPhases;
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::kLds];
@@ -616,8 +619,9 @@ int launch_a16_any(const A16GemmArgs& p, int max_row_tiles, hipStream_t stream) 
   return launch_a16<WF, MODE, 2>(p, max_row_tiles, stream);
 }
 
-A16GemmArgs a16_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L) {
+A16GemmArgs a16_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
   A16GemmArgs p = {};
+  p.gate = rows_gate(cfg, ws, L, n);
   p.topk = cfg.topk;
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
@@ -639,8 +643,8 @@ int gate_up(const A16GemmArgs& p, const afd_moe_cfg& cfg, int max_tiles, hipStre
 
 int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint16_t* x, const afd_job* rows_desc,
-                       hipStream_t stream) {
-  A16GemmArgs p = a16_args(cfg, ws, L);
+                       int32_t n, hipStream_t stream) {
+  A16GemmArgs p = a16_args(cfg, ws, L, n);
   p.a_rows = x;
   p.rows_desc = rows_desc;
   p.b_img = static_cast<const uint8_t*>(wt.w13);
@@ -654,8 +658,8 @@ int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
 }
 
 int launch_a16_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, hipStream_t stream) {
-  A16GemmArgs p = a16_args(cfg, ws, L);
+                    const afd_ws_layout& L, int32_t n, hipStream_t stream) {
+  A16GemmArgs p = a16_args(cfg, ws, L, n);
   p.a_img = ws + L.hq;
   p.b_img = static_cast<const uint8_t*>(wt.w2);
   p.b_scale = static_cast<const float*>(wt.s2);

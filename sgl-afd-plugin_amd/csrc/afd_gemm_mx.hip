@@ -56,6 +56,7 @@ struct MxGemmArgs {
   uint8_t* h_img;  // gate_up out: the down GEMM's A images [row tiles][N/256]
   ActParams act;   // gate_up: the activation
   uint16_t* y;     // down out: bf16 [np][N]
+  RowsGate gate;   // whether this launch or the few-rows GEMM runs
 };
 
 // Shape of the workgroup tile: 2 x WN wavefronts in two groups of WN (group g = rows
@@ -109,6 +110,7 @@ extern "C" __device__ v16f mfma_scale_f4_f8(v4i a, v8i b, v16f c, int cbsz, int 
 template <int MODE, int WN, bool kCont>
 __global__ __launch_bounds__(MxTile<WN>::kThreads) void mx_gemm_kernel(MxGemmArgs p) {
   static_assert(!kCont || MODE != kDown, "the continuous ring is gate_up's (down stages y in LDS)");
+  if (p.gate.large_skips()) return;
   using T = MxTile<WN>;
   constexpr int kBM = T::kBM, kBN = T::kBN, kStages = T::kStages, kStage = T::kStage;
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::kLds];
@@ -677,8 +679,9 @@ static int launch_mx_any(const MxGemmArgs& p, int max_row_tiles, hipStream_t str
 
 int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                       const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                      const afd_job* rows_desc, hipStream_t stream) {
+                      const afd_job* rows_desc, int32_t n, hipStream_t stream) {
   MxGemmArgs p;
+  p.gate = rows_gate(cfg, ws, L, n);
   p.a_img = nullptr;
   p.a_rows = xq;
   p.a_scales = static_cast<const uint8_t*>(xs);
@@ -703,8 +706,8 @@ int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint
 
 int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                    const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  (void)n;
   MxGemmArgs p;
+  p.gate = rows_gate(cfg, ws, L, n);
   p.act = act_params(cfg);
   p.a_img = ws + L.hq;
   p.a_rows = nullptr;

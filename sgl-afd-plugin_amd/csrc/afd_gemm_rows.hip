@@ -49,6 +49,7 @@ struct RowsArgs {
   const float* bs;           // FP8: block scales [E][N/128][K/128] (gate blocks, then up)
   const int32_t* sorted_pairs;
   const int32_t* counts;
+  RowsGate gate;
   int num_local;
   int K, N;
   uint32_t ntn_magic;  // div_magic(N / 256)
@@ -135,6 +136,7 @@ __global__ __launch_bounds__(256, 2) void rows_gemm_kernel(RowsArgs p) {
   constexpr bool kGU = MODE != kDown;
   constexpr int kBM = F::kBM;
   constexpr int kRows = 32 * R;
+  if (p.gate.few_skips()) return;
   const int ntn = p.N / kImgBRows;
   const int t = threadIdx.x, lane = t & 63, lr = lane & 31, lk = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -610,7 +612,10 @@ template <int FMT, int MODE>
 int launch_rows(const RowsArgs& p, int32_t n, int topk, hipStream_t stream) {
   constexpr int R = 2;
   // row groups of n tokens: at most one per pair, and one per expert plus one per 32 R pairs
-  const int64_t pairs = int64_t(n) * topk, most = p.num_local + pairs / (32 * R);
+  // (gated: of at most `limit` local pairs)
+  int64_t pairs = int64_t(n) * topk;
+  if (p.gate.pairs != nullptr && pairs > p.gate.limit) pairs = p.gate.limit;
+  const int64_t most = p.num_local + pairs / (32 * R);
   const int64_t groups = pairs < most ? pairs : most;
   hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, R>), dim3(static_cast<unsigned>(groups * (p.N / kImgBRows))),
                      dim3(256), 0, stream, p);
@@ -627,8 +632,9 @@ int launch_fmt(const RowsArgs& p, const afd_moe_cfg& cfg, int32_t n, hipStream_t
                                        : launch_rows<kF8, MODE>(p, n, cfg.topk, stream);
 }
 
-RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L) {
+RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
   RowsArgs p = {};
+  p.gate = rows_gate(cfg, ws, L, n);
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
   p.sorted_pairs = reinterpret_cast<const int32_t*>(ws + L.sorted_pairs);
@@ -639,20 +645,40 @@ RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L) 
 
 }  // namespace
 
-// The line lies where the large tiles catch up with every expert of the model local, as an FP8
-// rank of 64 experts has it (top-8, hidden 4096, inter 1536, large tiles -> few rows): at 37
-// rows per expert 278 -> 234 us (uniform routing) and 328 -> 283 (Zipf 1.2), at 64 rows 285 -> 339
-// and 343 -> 346. A rank that owns a quarter of the experts has a quarter of those rows (the
-// call does not know which share is local): 192 -> 162 us at the line, and the large tiles only
-// catch up at four times as many tokens.
-bool few_rows(const afd_moe_cfg& cfg, int32_t n) {
-  return int64_t(n) * cfg.topk <= int64_t(kFewRowsPerExpert) * cfg.num_local;
+// Pairs per local expert up to which the few-rows GEMMs run. The line lies where the large tiles
+// catch up (large tiles -> few rows): 64 FP8 experts, all local, hidden 4096, inter 1536, top-8: at
+// 37 pairs per expert 278 -> 234 us (uniform routing) and 328 -> 283 (Zipf 1.2), at 64 285 -> 339
+// and 343 -> 346; MXFP4 experts, hidden 4096, inter 2048: at 32 200 -> 189 us (uniform) and
+// 236 -> 222 (Zipf 1.2), at 48 210 -> 225 and 245 -> 259, with bf16 activations at 35 366 -> 270.
+constexpr int kFewRowsPerExpert = 40;
+// A call knows its own pairs, not how many of them are local: with at most 40 pairs per local
+// expert if all were, the few-rows GEMMs are launched alone. An MXFP4 rank that owns a quarter of
+// a model's experts has the line at four times as many tokens, so nearly up to there both forms
+// are launched and the router's count of local pairs decides between them: 64 of 256 experts, 512
+// tokens 233 -> 185 us, 750 tokens 237 -> 207 (Zipf 1.2), 194 -> 179 (uniform), with bf16
+// activations 512 tokens 334 -> 219, 1024 362 -> 274. Where the large tiles then run after all, the
+// two launches that return at once cost 4 to 5 us (2% at 1200 tokens), which is why this ends a
+// little before a quarter. FP8 experts gain nothing there (32 of 128 experts, 512 tokens: 68 -> 74
+// us) and take the large tiles.
+constexpr int kGatedRowsPerExpert = 140;
+RowsForm rows_form(const afd_moe_cfg& cfg, int32_t n) {
+  const int64_t pairs = int64_t(n) * cfg.topk;
+  if (pairs <= int64_t(kFewRowsPerExpert) * cfg.num_local) return kRowsFew;
+  return cfg.weight_fmt == AFD_W_MXFP4 && pairs <= int64_t(kGatedRowsPerExpert) * cfg.num_local ? kRowsBoth
+                                                                                               : kRowsLarge;
+}
+
+RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
+  if (rows_form(cfg, n) != kRowsBoth) return RowsGate{nullptr, 0};
+  // offsets[num_local]: the call's local pairs
+  return RowsGate{reinterpret_cast<const int32_t*>(ws + L.offsets) + cfg.num_local,
+                  kFewRowsPerExpert * cfg.num_local};
 }
 
 int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                         const afd_ws_layout& L, const void* x, const void* xs, const afd_job* rows_desc,
                         int32_t n, hipStream_t stream) {
-  RowsArgs p = rows_args(cfg, ws, L);
+  RowsArgs p = rows_args(cfg, ws, L, n);
   p.a = static_cast<const uint8_t*>(x);
   p.as = static_cast<const uint8_t*>(xs);
   p.rows_desc = rows_desc;
@@ -669,7 +695,7 @@ int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, ui
 
 int launch_rows_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                      const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  RowsArgs p = rows_args(cfg, ws, L);
+  RowsArgs p = rows_args(cfg, ws, L, n);
   p.a = ws + L.hq;
   p.as = ws + L.hs;
   p.b = static_cast<const uint8_t*>(wt.w2);

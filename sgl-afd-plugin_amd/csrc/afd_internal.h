@@ -131,7 +131,7 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
 // descriptor's xq / xs when the kernel runs.
 int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                       const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                      const afd_job* rows_desc, hipStream_t stream);
+                      const afd_job* rows_desc, int32_t n, hipStream_t stream);
 int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                    const afd_ws_layout& L, int32_t n, hipStream_t stream);
 
@@ -140,9 +140,9 @@ int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t
 // that job descriptor's x, read when the kernel runs.
 int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint16_t* x, const afd_job* rows_desc,
-                       hipStream_t stream);
+                       int32_t n, hipStream_t stream);
 int launch_a16_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, hipStream_t stream);
+                    const afd_ws_layout& L, int32_t n, hipStream_t stream);
 
 // Grouped FP8 128x128-block GEMMs (afd_gemm_fp8.hip).
 int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
@@ -152,9 +152,19 @@ int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_
                     const afd_ws_layout& L, int32_t n, hipStream_t stream);
 
 // Grouped GEMMs for few tokens per expert (afd_gemm_rows.hip), every format; the same results bit
-// for bit. few_rows: whether a call of n tokens takes them.
-constexpr int kFewRowsPerExpert = 40;
-bool few_rows(const afd_moe_cfg& cfg, int32_t n);
+// for bit. Which GEMMs a call of n tokens launches: the few-rows ones, the large-tile ones, or
+// both, gated: then both read the call's local pairs and all but one form return at once.
+enum RowsForm { kRowsLarge = 0, kRowsFew = 1, kRowsBoth = 2 };
+RowsForm rows_form(const afd_moe_cfg& cfg, int32_t n);
+// The gate of a GEMM launch: it runs if the call's local pairs are (few) at most `limit` or
+// (large) above it; pairs == nullptr: it runs.
+struct RowsGate {
+  const int32_t* pairs;
+  int limit;
+  __device__ __forceinline__ bool few_skips() const { return pairs != nullptr && *pairs > limit; }
+  __device__ __forceinline__ bool large_skips() const { return pairs != nullptr && *pairs <= limit; }
+};
+RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n);
 // x / xs: the token rows in the activation format (quantized, or bf16 with xs null); with
 // rows_desc != nullptr they are read from that job descriptor when the kernel runs.
 int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,

@@ -2,8 +2,9 @@
 //
 // Integer work on a 4*n*k-byte id array (HBM/latency bound). Two launches, or with few pairs one
 // (each workgroup of the second then counts the pairs by itself, at most 16 loads a thread, which
-// overlap, while workgroups beside it quantize; 15 -> 10 us of routing for 24 tokens of 64 FP8
-// experts):
+// overlap, while workgroups beside it quantize; with the shared fill 15.4 -> 5.0 us of routing for
+// 24 tokens of 64 FP8 experts, 12.3 -> 7.3 for 2400 pairs of an MXFP4 rank; two launches of 4136
+// pairs take 10.8, and one launch comes near that at kFusedPairs):
 //   1. route_prep:    workgroup c < chunks histograms chunk c of the flat pair array by local
 //                     expert (LDS atomics; counts are order-free); with the expert call, the
 //                     remaining workgroups quantize the activations meanwhile (afd_quant_dev.h).
@@ -11,13 +12,12 @@
 //                     by expert, [E][kMaxChunks], so each thread's run of chunk counts is a few
 //                     16-byte loads issued together) to get each expert's count, its own chunk's
 //                     base per expert and the block_m-padded expert offsets (a wavefront scan);
-//                     workgroup 0 also writes
-//                     counts, offsets, padded offsets, the row-tile table and the tile count;
-//                     the -1 fill of padding rows is dealt to all workgroups. It then walks its pairs in flat order, 256 at
-//                     a time; a pair's rank among equal keys inside its wavefront comes from 9
-//                     ballots (one per key bit), across wavefronts from LDS counts, so the
-//                     placement is the stable order (ascending flat index inside each expert)
-//                     bit for bit.
+//                     workgroup 0 also writes counts, offsets, padded offsets, the row-tile
+//                     table and the tile count; the -1 fill of padding rows is dealt to all
+//                     workgroups. It then walks its pairs in flat order, 256 at a time; a pair's
+//                     rank among equal keys inside its wavefront comes from 9 ballots (one per
+//                     key bit), across wavefronts from LDS counts, so the placement is the stable
+//                     order (ascending flat index inside each expert) bit for bit.
 #include "afd_common.h"
 #include "afd_internal.h"
 #include "afd_quant_dev.h"

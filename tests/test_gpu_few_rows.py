@@ -4,6 +4,9 @@ format, at the sizes where they can go wrong: expert counts around the 32-row bl
 with no row, one K stage and K stages that do not fill the register ring, one and several weight
 image columns, and an expert count that is not a multiple of the 4 a lane looks up.
 
+Above that, up to GATED tokens per local expert, an MXFP4 call launches both the few-rows and
+the large-tile GEMMs and the number of local pairs decides on the GPU; both outcomes are run.
+
 The large-tile GEMMs and the few-rows GEMMs feed every accumulator the same products in the
 same order, so the same tokens inside a call large enough for the large tiles must give the
 same bits; against the oracle the bar is that of the other layer tests (rel-L2 1e-2: the same
@@ -26,8 +29,10 @@ pytestmark = pytest.mark.gpu
 REL_L2_TOL = 1e-2
 # rows of the first experts; the others get none
 COUNTS = [1, 0, 31, 32, 33, 63, 64, 65, 127, 128, 129, 0, 2, 255, 256, 257, 7]
-# tokens per local expert up to which a call takes the few-rows GEMMs (topk 1 here)
+# tokens per local expert (topk 1 here) up to which a call takes the few-rows GEMMs, and up to which
+# the number of local pairs decides
 FEW_ROWS = 40
+GATED = 140
 
 
 def ids_for(counts, num_local, total, gen):
@@ -53,14 +58,15 @@ def ids_for(counts, num_local, total, gen):
 )
 def test_few_rows_match_large_tiles(hidden, inter, activation, fmt, act):
     num_local = 42
-    n, more = sum(COUNTS) + 5, FEW_ROWS * num_local + 1
-    assert n <= FEW_ROWS * num_local
+    n, more = sum(COUNTS) + 5, GATED * num_local + 1
+    assert n <= FEW_ROWS * num_local < n + 300 and 3000 + n <= GATED * num_local
     say(f"few rows H={hidden} I={inter} {activation} {fmt} {act} n={n}")
     gen = W.generator("cpu", 17)
     x = W.tokens(n + more, hidden, gen, "cpu")
     w = torch.rand(n + more, 1, generator=gen) + 0.25
     ids = torch.cat([ids_for(COUNTS, num_local, n, gen),
-                     torch.randint(0, num_local + 1, (more, 1), generator=gen, dtype=torch.int32)])
+                     torch.randint(0, num_local, (more, 1), generator=gen, dtype=torch.int32)])
+    ids[n:n + 300] = num_local
     w13, w2 = W.expert_weights(num_local, hidden, inter, gen, "cpu")
     pack = pack_mxfp4_experts if fmt == "mxfp4" else pack_fp8_block_experts
     kw, oact = {}, {}
@@ -78,7 +84,9 @@ def test_few_rows_match_large_tiles(hidden, inter, activation, fmt, act):
         return bits16(out)
 
     few = call(n)
-    assert np.array_equal(few, call(n + more)[:n])
+    # few local pairs among more tokens, more local pairs, and beyond the range of either
+    for m in (n + 300, 3000 + n, n + more):
+        assert np.array_equal(few, call(m)[:n]), m
     quant = "bf16" if act == "bf16" else "mxfp8" if fmt == "mxfp4" else "fp8_1x128"
     ref = OX.moe_ffn(x[:n], ids[:n].numpy(), w[:n].numpy(), *deq_weights(w13, w2, fmt), 0, act=quant, **oact)
     err = rel_l2(F.bf16_to_f32(few), F.bf16_to_f32(ref))
