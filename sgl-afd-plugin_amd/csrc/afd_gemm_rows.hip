@@ -5,10 +5,10 @@
 // decode step occupy 112 of 256 CUs, 38 experts take two rounds) and pay a barrier every half
 // stage.
 //
-// Split: a workgroup of 4 wavefronts owns a row group (at most 64 rows of one expert) x the 256
+// Split: a workgroup of 4 wavefronts owns a row group (at most 32 R = 32 or 64 rows of one expert) x the 256
 // weight rows of one image column; wavefront w streams its 64 rows (gate_up: 32 gate and the
 // matching 32 up rows; 4 KiB of each image) over the whole K from HBM into registers, several K
-// stages of 128 ahead, so 256-column items fill the chip and two workgroups a CU keep 70-100 KB
+// stages of 128 ahead, so 256-column items fill the chip and 2 or 3 workgroups a CU keep 70-150 KB
 // of weights in flight. A stage passes through LDS on its way to the matrix instructions: the
 // weights through the wavefront's own area, which lets the loads be contiguous kilobytes (read in
 // fragment order, half a line a load, non-temporal loads reach 5.3 TB/s here and default ones
@@ -123,15 +123,17 @@ __device__ __forceinline__ v8i join(v4i lo, v4i hi) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// K stages in flight for NB 32-row blocks: as many as 256 registers hold beside the 32 NB
-// accumulators (17 or 32 registers of weights and 5 or 8 per row block of activations a stage)
-template <int FMT, int NB>
+// K stages in flight for NB 32-row blocks in groups of R: as many as the registers (256, or 168 for
+// three workgroups a CU with R = 1) hold beside the 32 NB accumulators (17 or 32 registers of
+// weights and 5 or 8 per row block of activations a stage)
+template <int FMT, int NB, int R>
 constexpr int depth() {
+  if (R == 1) return FMT == kMx8 ? 4 : FMT == kMx16 ? 3 : 2;
   return FMT == kMx8 ? 4 : FMT == kMx16 ? (NB == 1 ? 4 : 3) : NB == 1 ? 3 : 2;
 }
 
 template <int FMT, int MODE, int R>
-__global__ __launch_bounds__(256, 2) void rows_gemm_kernel(RowsArgs p) {
+__global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs p) {
   using F = Fmt<FMT>;
   constexpr bool kGU = MODE != kDown;
   constexpr int kBM = F::kBM;
@@ -214,7 +216,7 @@ __global__ __launch_bounds__(256, 2) void rows_gemm_kernel(RowsArgs p) {
   // rows [r0, live) of the tile as NB blocks of 32
   auto pass = [&](auto nb_c) __attribute__((always_inline)) {
     constexpr int NB = decltype(nb_c)::value;
-    constexpr int D = depth<FMT, NB>();
+    constexpr int D = depth<FMT, NB, R>();
     struct Stage {
       v4i w[F::kImgs][4];  // the wavefront's 4 KiB of each image, 1 KiB a load
       uint32_t sw;         // MXFP4: the scale word of weight row 64 w + lane
@@ -608,17 +610,26 @@ __global__ __launch_bounds__(256, 2) void rows_gemm_kernel(RowsArgs p) {
   pass(std::integral_constant<int, 1>{});
 }
 
+// Groups of 32 rows run three workgroups a CU instead of two, groups of 64 read the weights of an
+// expert of 33 to 64 rows once: 32 while few experts have more rows. At most 16 pairs per expert:
+// -6 to +0.6% over the four formats and two routings (64 FP8 experts, bf16 activations, 8 tokens
+// 121 -> 117 us; 32 local of hidden 2048, 64 tokens 46 -> 43); at 25 219 -> 236 us (FP8 experts, all
+// local), at 37 224 -> 353.
+constexpr int kNarrowRowsPerExpert = 16;
 template <int FMT, int MODE>
 int launch_rows(const RowsArgs& p, int32_t n, int topk, hipStream_t stream) {
-  constexpr int R = 2;
-  // row groups of n tokens: at most one per pair, and one per expert plus one per 32 R pairs
-  // (gated: of at most `limit` local pairs)
+  const int cols = p.N / kImgBRows;
   int64_t pairs = int64_t(n) * topk;
+  const bool narrow = pairs <= int64_t(kNarrowRowsPerExpert) * p.num_local;
+  // row groups of n tokens: at most one per pair, and one per expert plus one per full group
+  // (gated: of at most `limit` local pairs)
   if (p.gate.pairs != nullptr && pairs > p.gate.limit) pairs = p.gate.limit;
-  const int64_t most = p.num_local + pairs / (32 * R);
-  const int64_t groups = pairs < most ? pairs : most;
-  hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, R>), dim3(static_cast<unsigned>(groups * (p.N / kImgBRows))),
-                     dim3(256), 0, stream, p);
+  const int64_t most = p.num_local + pairs / (narrow ? 32 : 64);
+  const dim3 grid(static_cast<unsigned>((pairs < most ? pairs : most) * cols));
+  if (narrow)
+    hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, 1>), grid, dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, 2>), grid, dim3(256), 0, stream, p);
   AFD_CHECK_LAUNCH();
   return AFD_OK;
 }

@@ -1,6 +1,6 @@
 """GPU: the few-rows GEMMs (calls with few tokens per expert), every weight and activation
 format, at the sizes where they can go wrong: expert counts around the 32-row blocks, the
-64-row groups and the row tiles (128, or 256 for FP8 block weights with fp8 activations), experts
+32- and 64-row groups and the row tiles (128, or 256 for FP8 block weights with fp8 activations), experts
 with no row, one K stage and K stages that do not fill the register ring, one and several weight
 image columns, and an expert count that is not a multiple of the 4 a lane looks up.
 
@@ -49,18 +49,21 @@ def ids_for(counts, num_local, total, gen):
 @pytest.mark.parametrize("act", ["fp8", "bf16"])
 @pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block"])
 @pytest.mark.parametrize(
-    "hidden,inter,activation",
+    "num_local,hidden,inter,activation",
     [
-        (256, 128, "silu"),  # 2 and 1 K stages, one image column in each GEMM
-        (768, 384, "silu_limit"),  # 6 and 3 K stages, 3 columns
-        (1280, 1152, "situ"),  # 10 and 9 K stages
+        # groups of 64 rows
+        (42, 256, 128, "silu"),  # 2 and 1 K stages, one image column in each GEMM
+        (42, 768, 384, "silu_limit"),  # 6 and 3 K stages, 3 columns
+        (42, 1280, 1152, "situ"),  # 10 and 9 K stages
+        # groups of 32 rows (the n + 300 tokens below: of 64)
+        (101, 256, 128, "situ"),
+        (101, 512, 384, "silu"),
     ],
 )
-def test_few_rows_match_large_tiles(hidden, inter, activation, fmt, act):
-    num_local = 42
+def test_few_rows_match_large_tiles(num_local, hidden, inter, activation, fmt, act):
     n, more = sum(COUNTS) + 5, GATED * num_local + 1
-    assert n <= FEW_ROWS * num_local < n + 300 and 3000 + n <= GATED * num_local
-    say(f"few rows H={hidden} I={inter} {activation} {fmt} {act} n={n}")
+    assert n <= FEW_ROWS * num_local < 3000 + n <= GATED * num_local
+    say(f"few rows E={num_local} H={hidden} I={inter} {activation} {fmt} {act} n={n}")
     gen = W.generator("cpu", 17)
     x = W.tokens(n + more, hidden, gen, "cpu")
     w = torch.rand(n + more, 1, generator=gen) + 0.25
@@ -84,7 +87,8 @@ def test_few_rows_match_large_tiles(hidden, inter, activation, fmt, act):
         return bits16(out)
 
     few = call(n)
-    # few local pairs among more tokens, more local pairs, and beyond the range of either
+    # a few more tokens without a local expert (42 experts: the local pairs decide), more local pairs
+    # (the large tiles, by the same decision), and beyond its range
     for m in (n + 300, 3000 + n, n + more):
         assert np.array_equal(few, call(m)[:n]), m
     quant = "bf16" if act == "bf16" else "mxfp8" if fmt == "mxfp4" else "fp8_1x128"
