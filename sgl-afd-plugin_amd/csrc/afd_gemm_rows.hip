@@ -5,8 +5,8 @@
 // decode step occupy 112 of 256 CUs, 38 experts take two rounds) and pay a barrier every half
 // stage.
 //
-// Split: a workgroup of 4 wavefronts owns a row group (at most 32 R = 32 or 64 rows of one expert) x the 256
-// weight rows of one image column; wavefront w streams its 64 rows (gate_up: 32 gate and the
+// Split: a workgroup of 4 wavefronts owns a row group (at most 32 R = 32 or 64 rows of one
+// expert) x the 256 weight rows of one image column; wavefront w streams its 64 rows (gate_up: 32 gate and the
 // matching 32 up rows; 4 KiB of each image) over the whole K from HBM into registers, several K
 // stages of 128 ahead, so 256-column items fill the chip and 2 or 3 workgroups a CU keep 70-150 KB
 // of weights in flight. A stage passes through LDS on its way to the matrix instructions: the
@@ -16,10 +16,11 @@
 // a quarter each and share (each wavefront reading its own copy from L2 was as fast at 1 to 16
 // rows per expert and 20 to 35% slower at 32 to 64).
 //
-// Measured against the large-tile kernels (whole expert call, cold caches): hidden 4096, inter
-// 2048, 64 of 256 MXFP4 experts local, top-8, Zipf(1.2): 8 tokens 75 -> 47 us, 64 tokens 151 -> 106,
-// 300 tokens 188 -> 165 (fp8 activations); 128 tokens 233 -> 134 (bf16 activations). Hidden 4096,
-// inter 1536, 64 FP8-block experts, top-8: 16 tokens 254 -> 191 us, 128 tokens 275 -> 216. The
+// Measured against the large-tile kernels (whole expert call, cold caches, with the router's one
+// launch for few pairs, which gives about 5 to 10 us of it): hidden 4096, inter 2048, 64 of 256
+// MXFP4 experts local, top-8, Zipf(1.2): 8 tokens 75 -> 42 us, 64 tokens 151 -> 100, 300 tokens
+// 188 -> 160 (fp8 activations); 128 tokens 233 -> 125 (bf16 activations). Hidden 4096, inter 1536,
+// 64 FP8-block experts, top-8, uniform routing: 8 tokens 226 -> 135 us, 128 tokens 275 -> 203. The
 // reads then run at 5.0 to 5.5 TB/s.
 //
 // Every accumulator sees the MFMAs of the large-tile kernels, in their order, with their scale
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
 #pragma unroll
         for (int h = 0; h < F::kALoads; ++h) f.a[i][h] = load_global<v4i>(base, ao[i][h]);
         if constexpr (FMT == kMx8)
-          f.sa[i] = kGU ? load_global<uint16_t>(scalar_base(a_scales + int64_t(kt) * 4), so[i]) : load_global<uint16_t>(base, so[i]);
+          f.sa[i] = load_global<uint16_t>(kGU ? scalar_base(a_scales + int64_t(kt) * 4) : base, so[i]);
         else if constexpr (FMT == kF8)
           f.sa[i] = load_global<uint32_t>(
               scalar_base(a_scales + (kGU ? int64_t(kt) * 4 : (int64_t(mt) * kb_n + kt) * (kBM * 4))), so[i]);
