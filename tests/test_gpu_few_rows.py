@@ -100,3 +100,33 @@ def test_few_rows_match_large_tiles(num_local, hidden, inter, activation, fmt, a
     for e in (0, num_local - 1):
         ids[:1] = e
         assert np.array_equal(call(1), call(n + more)[:1]), e
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block"])
+@pytest.mark.parametrize("num_local,counts", [(42, {40: 1601}), (101, {0: 65, 3: 32, 100: 1500})])
+def test_concentrated_rows_match_large_tiles(num_local, counts, fmt, act):
+    """One expert with most of a few-rows call's pairs: 26 groups of 64 rows (47 of 32 with 101
+    experts), which read its weights through the cache while an expert of one group streams past
+    it; the same bits as inside a call of the large tiles."""
+    n, more = sum(counts.values()), GATED * num_local + 1
+    assert n <= FEW_ROWS * num_local
+    say(f"concentrated E={num_local} {fmt} {act} counts={counts}")
+    gen = W.generator("cpu", 23)
+    x = W.tokens(n + more, 512, gen, "cpu")
+    w = torch.rand(n + more, 1, generator=gen) + 0.25
+    ids = torch.cat([ids_for([counts.get(e, 0) for e in range(num_local)], num_local, n, gen),
+                     torch.randint(0, num_local, (more, 1), generator=gen, dtype=torch.int32)])
+    w13, w2 = W.expert_weights(num_local, 512, 384, gen, "cpu")
+    pack = pack_mxfp4_experts if fmt == "mxfp4" else pack_fp8_block_experts
+    experts = AfdExperts(num_local + 1, 1, 0, range(num_local), pack(w13, w2, device=dev()), n_max=n + more,
+                         act_format="bf16" if act == "bf16" else None)
+
+    def call(m):
+        out = experts(x[:m].to(dev()), StandardTopKOutput(w[:m].to(dev()), ids[:m].to(dev())))
+        torch.cuda.synchronize()
+        return bits16(out)
+
+    few = call(n)
+    assert np.isfinite(F.bf16_to_f32(few)).all()
+    assert np.array_equal(few, call(n + more)[:n])
