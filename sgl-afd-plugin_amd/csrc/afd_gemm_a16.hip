@@ -167,8 +167,7 @@ __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A
   using T = A16Tile<WF, WN>;
   using F = typename T::F;
   constexpr bool kFp8 = WF == kWFp8;
-  if constexpr (!kFp8)  // FP8 weights: never gated
-    if (p.gate.large_skips()) return;
+  if (p.gate.large_skips()) return;
   constexpr int kBM = T::kBM, kBN = T::kBN, kStages = T::kStages, kStage = T::kStage;
   constexpr int kStageK = T::kStageK, kPhases = T::kPhases;
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::kLds];

@@ -68,6 +68,7 @@ struct Fp8GemmArgs {
   uint8_t* hq;    // gate_up out: h images [row tiles][N/2/64]
   float* hs;      // gate_up out: h scales [row tiles][N/2/128][128]
   uint16_t* y;    // down out: bf16 [np][N]
+  RowsGate gate;  // whether this launch or the few-rows GEMM runs
 };
 
 // The tile: 256 activation rows (two 128-row blocks of one expert: the router pads this
@@ -127,6 +128,7 @@ __device__ __forceinline__ float load_uniform(const float* p) {
 
 template <int MODE>
 __global__ __launch_bounds__(Tile::kThreads) void fp8_gemm_kernel(Fp8GemmArgs p) {
+  if (p.gate.large_skips()) return;
   using T = Tile;
   constexpr int kBM = T::kBM, kBN = T::kBN, kStages = T::kStages, kStage = T::kStage;
   constexpr bool kGU = MODE != kDown;
@@ -678,8 +680,9 @@ static int launch(const Fp8GemmArgs& p, int max_row_tiles, hipStream_t stream) {
   return AFD_OK;
 }
 
-static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L) {
+static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
   Fp8GemmArgs p = {};
+  p.gate = rows_gate(cfg, ws, L, n);
   p.topk = cfg.topk;
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
@@ -695,8 +698,8 @@ static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws
 
 int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                       const afd_job* rows_desc, hipStream_t stream) {
-  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L);
+                       const afd_job* rows_desc, int32_t n, hipStream_t stream) {
+  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, n);
   p.a = xq;
   p.as = static_cast<const float*>(xs);
   p.rows_desc = rows_desc;
@@ -713,8 +716,7 @@ int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
 
 int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                     const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  (void)n;
-  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L);
+  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, n);
   p.a = ws + L.hq;
   p.as = reinterpret_cast<const float*>(ws + L.hs);
   p.b = static_cast<const uint8_t*>(wt.w2);

@@ -620,29 +620,21 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
     }
     pass(std::integral_constant<int, 1>{}, once_c);
   };
-  if (rows <= kRows)  // the expert's only group
+  if (__builtin_expect(rows <= kRows, 1))  // the expert's only group (its code comes first)
     pass_rows(std::true_type{});
   else
     pass_rows(std::false_type{});
 }
 
-// Groups of 32 rows run three workgroups a CU instead of two, groups of 64 read the weights of an
-// expert of 33 to 64 rows once: 32 while few experts have more rows. At most 16 pairs per expert:
-// -6 to +0.6% over the four formats and two routings (64 FP8 experts, bf16 activations, 8 tokens
-// 121 -> 117 us; 32 local of hidden 2048, 64 tokens 46 -> 43); at 25 219 -> 236 us (FP8 experts, all
-// local), at 37 224 -> 353.
-constexpr int kNarrowRowsPerExpert = 16;
 template <int FMT, int MODE>
-int launch_rows(const RowsArgs& p, int32_t n, int topk, hipStream_t stream) {
+int launch_rows(const RowsArgs& p, const RowsPlan& plan, int64_t pairs, hipStream_t stream) {
   const int cols = p.N / kImgBRows;
-  int64_t pairs = int64_t(n) * topk;
-  const bool narrow = pairs <= int64_t(kNarrowRowsPerExpert) * p.num_local;
-  // row groups of n tokens: at most one per pair, and one per expert plus one per full group
-  // (gated: of at most `limit` local pairs)
-  if (p.gate.pairs != nullptr && pairs > p.gate.limit) pairs = p.gate.limit;
-  const int64_t most = p.num_local + pairs / (narrow ? 32 : 64);
+  // row groups of so many pairs: at most one per pair, and one per expert plus one per full group
+  // (gated: of at most max_pairs local pairs)
+  if (plan.form == kRowsBoth && pairs > plan.max_pairs) pairs = plan.max_pairs;
+  const int64_t most = p.num_local + (pairs >> plan.group_shift);
   const dim3 grid(static_cast<unsigned>((pairs < most ? pairs : most) * cols));
-  if (narrow)
+  if (plan.group_shift == 5)
     hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, 1>), grid, dim3(256), 0, stream, p);
   else
     hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, 2>), grid, dim3(256), 0, stream, p);
@@ -652,11 +644,13 @@ int launch_rows(const RowsArgs& p, int32_t n, int topk, hipStream_t stream) {
 
 template <int MODE>
 int launch_fmt(const RowsArgs& p, const afd_moe_cfg& cfg, int32_t n, hipStream_t stream) {
+  const RowsPlan plan = rows_plan(cfg, n);
+  const int64_t pairs = int64_t(n) * cfg.topk;
   if (cfg.act_fmt == AFD_A_BF16)
-    return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx16, MODE>(p, n, cfg.topk, stream)
-                                         : launch_rows<kF16, MODE>(p, n, cfg.topk, stream);
-  return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx8, MODE>(p, n, cfg.topk, stream)
-                                       : launch_rows<kF8, MODE>(p, n, cfg.topk, stream);
+    return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx16, MODE>(p, plan, pairs, stream)
+                                         : launch_rows<kF16, MODE>(p, plan, pairs, stream);
+  return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx8, MODE>(p, plan, pairs, stream)
+                                       : launch_rows<kF8, MODE>(p, plan, pairs, stream);
 }
 
 RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
@@ -672,34 +666,9 @@ RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, 
 
 }  // namespace
 
-// Pairs per local expert up to which the few-rows GEMMs run. The line lies where the large tiles
-// catch up (large tiles -> few rows): 64 FP8 experts, all local, hidden 4096, inter 1536, top-8: at
-// 37 pairs per expert 278 -> 234 us (uniform routing) and 328 -> 283 (Zipf 1.2), at 64 285 -> 339
-// and 343 -> 346; MXFP4 experts, hidden 4096, inter 2048: at 32 200 -> 189 us (uniform) and
-// 236 -> 222 (Zipf 1.2), at 48 210 -> 225 and 245 -> 259, with bf16 activations at 35 366 -> 270.
-constexpr int kFewRowsPerExpert = 40;
-// A call knows its own pairs, not how many of them are local: with at most 40 pairs per local
-// expert if all were, the few-rows GEMMs are launched alone. An MXFP4 rank that owns a quarter of
-// a model's experts has the line at four times as many tokens, so nearly up to there both forms
-// are launched and the router's count of local pairs decides between them: 64 of 256 experts, 512
-// tokens 233 -> 185 us, 750 tokens 237 -> 207 (Zipf 1.2), 194 -> 179 (uniform), with bf16
-// activations 512 tokens 334 -> 219, 1024 362 -> 274. Where the large tiles then run after all, the
-// two launches that return at once cost 4 to 5 us (2% at 1200 tokens), which is why this ends a
-// little before a quarter. FP8 experts gain nothing there (32 of 128 experts, 512 tokens: 68 -> 74
-// us) and take the large tiles.
-constexpr int kGatedRowsPerExpert = 140;
-RowsForm rows_form(const afd_moe_cfg& cfg, int32_t n) {
-  const int64_t pairs = int64_t(n) * cfg.topk;
-  if (pairs <= int64_t(kFewRowsPerExpert) * cfg.num_local) return kRowsFew;
-  return cfg.weight_fmt == AFD_W_MXFP4 && pairs <= int64_t(kGatedRowsPerExpert) * cfg.num_local ? kRowsBoth
-                                                                                               : kRowsLarge;
-}
-
 RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
-  if (rows_form(cfg, n) != kRowsBoth) return RowsGate{nullptr, 0};
-  // offsets[num_local]: the call's local pairs
-  return RowsGate{reinterpret_cast<const int32_t*>(ws + L.offsets) + cfg.num_local,
-                  kFewRowsPerExpert * cfg.num_local};
+  if (rows_plan(cfg, n).form != kRowsBoth) return RowsGate{nullptr};
+  return RowsGate{reinterpret_cast<const int32_t*>(call_counters(ws, L)) + kRowsFewWord};
 }
 
 int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/afd.h"
+#include "afd_rows_rule.h"
 
 namespace afd {
 
@@ -84,12 +85,14 @@ __device__ __forceinline__ JobIn resolve_job(JobIn j) {
   return j;
 }
 
-// Counter words of one call, in the workspace's num_tiles slot (num_tiles is word 0). Returning
+// Counter words of one call, in the workspace's num_tiles slot (num_tiles is word 0, the router's
+// choice of the GEMMs word 1: 1 few rows, 0 large tiles, written if both are launched). Returning
 // atomics on one cache line serialize (~10 ns each), so the counters that many workgroups hit
 // at once each have a 256-byte line of their own: line l (l < kCounterLines) starts at word
 // kLineWord0 + l * kLineStride and holds, in its words 0 / 1 / 2, the reply's group counter l,
 // the gate_up GEMM's tile counter of XCD l and the down GEMM's (l < 8). The routing launch
 // zeroes those words and kArriveWord before any later launch of the call uses them.
+constexpr int kRowsFewWord = 1;
 constexpr int kArriveWord = 32;  // the reply's arrive counter (one count per group)
 constexpr int kLineWord0 = 64, kLineStride = 64, kCounterLines = 32;
 constexpr int kArriveGroups = kCounterLines, kArriveGroupWord0 = kLineWord0, kArriveGroupStride = kLineStride;
@@ -147,22 +150,17 @@ int launch_a16_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_
 // Grouped FP8 128x128-block GEMMs (afd_gemm_fp8.hip).
 int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                       const afd_job* rows_desc, hipStream_t stream);
+                       const afd_job* rows_desc, int32_t n, hipStream_t stream);
 int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                     const afd_ws_layout& L, int32_t n, hipStream_t stream);
 
 // Grouped GEMMs for few tokens per expert (afd_gemm_rows.hip), every format; the same results bit
-// for bit. Which GEMMs a call of n tokens launches: the few-rows ones, the large-tile ones, or
-// both, gated: then both read the call's local pairs and all but one form return at once.
-enum RowsForm { kRowsLarge = 0, kRowsFew = 1, kRowsBoth = 2 };
-RowsForm rows_form(const afd_moe_cfg& cfg, int32_t n);
-// The gate of a GEMM launch: it runs if the call's local pairs are (few) at most `limit` or
-// (large) above it; pairs == nullptr: it runs.
+// for bit. Which GEMMs a call of n tokens launches: rows_plan (afd_rows_rule.h).
+// The gate of a GEMM launch: it runs if the router chose its form; few == nullptr: it runs.
 struct RowsGate {
-  const int32_t* pairs;
-  int limit;
-  __device__ __forceinline__ bool few_skips() const { return pairs != nullptr && *pairs > limit; }
-  __device__ __forceinline__ bool large_skips() const { return pairs != nullptr && *pairs <= limit; }
+  const int32_t* few;
+  __device__ __forceinline__ bool few_skips() const { return few != nullptr && *few == 0; }
+  __device__ __forceinline__ bool large_skips() const { return few != nullptr && *few != 0; }
 };
 RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n);
 // x / xs: the token rows in the activation format (quantized, or bf16 with xs null); with

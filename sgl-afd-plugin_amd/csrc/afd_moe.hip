@@ -388,7 +388,7 @@ static int moe_ffn_impl(const afd_moe_cfg* cfg, const afd_expert_weights* weight
                             ev && ev[1] ? static_cast<hipEvent_t>(ev[1]) : nullptr);
     if (st != AFD_OK) return st;
     if ((st = mark(2)) != AFD_OK) return st;
-    const RowsForm form = rows_form(*cfg, n);
+    const int form = rows_plan(*cfg, n).form;
     const uint16_t* rows = staged_x != nullptr ? staged_x : job.x;
     const uint8_t* aq = quantized ? xq : wsb + L.xq;
     const void* as = quantized ? xs : static_cast<const void*>(wsb + L.xs);
@@ -399,7 +399,7 @@ static int moe_ffn_impl(const afd_moe_cfg* cfg, const afd_expert_weights* weight
     if (form != kRowsFew && st == AFD_OK)
       st = a16  ? launch_a16_gate_up(*cfg, *weights, wsb, L, rows, rows_desc, n, s)
            : mx ? launch_mx_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, n, s)
-                : launch_fp8_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, s);
+                : launch_fp8_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, n, s);
     if (st != AFD_OK || (st = mark(3)) != AFD_OK) return st;
     if (form != kRowsLarge) st = launch_rows_down(*cfg, *weights, wsb, L, n, s);
     if (form != kRowsFew && st == AFD_OK)

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
     const int32_t* __restrict__ hist, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ poff, int32_t* __restrict__ sorted_pairs,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ tile_expert,
-    int32_t* __restrict__ num_tiles, PrepQuant pq, uint32_t* __restrict__ counters) {
+    int32_t* __restrict__ num_tiles, PrepQuant pq, RowsPlan plan, uint32_t* __restrict__ counters) {
   const JobIn job = resolve_job(jin);
   if constexpr (kFused) {
     if (blockIdx.x == 0) zero_counters(counters);
@@ -215,6 +215,24 @@ __global__ __launch_bounds__(kRouteThreads) void route_scatter_kernel(
         num_tiles[0] = ip / block_m;
       }
     }
+  } else if (plan.form == kRowsBoth && c == 0 && t < 128) {
+    // beside it, another wavefront: the choice of the GEMMs
+    int pairs_here = 0, groups = 0, with_rows = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ex = lane * 4 + i;
+      const int n_e = ex < num_local ? tot[ex] : 0;
+      pairs_here += n_e;
+      groups += (n_e + (1 << plan.group_shift) - 1) >> plan.group_shift;
+      with_rows += n_e > 0;
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      pairs_here += __shfl_xor(pairs_here, d);
+      groups += __shfl_xor(groups, d);
+      with_rows += __shfl_xor(with_rows, d);
+    }
+    if (lane == 0) counters[kRowsFewWord] = rows_few(plan, pairs_here, groups, with_rows);
   }
   __syncthreads();
   for (int ex = t; ex < num_local; ex += kRouteThreads) run[ex] += pof[ex];
@@ -299,7 +317,7 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
                        reinterpret_cast<int32_t*>(ws + L.sorted_pairs),
                        reinterpret_cast<int32_t*>(ws + L.pair_pos),
                        reinterpret_cast<int32_t*>(ws + L.tile_expert),
-                       reinterpret_cast<int32_t*>(ws + L.num_tiles), pq, counters);
+                       reinterpret_cast<int32_t*>(ws + L.num_tiles), pq, rows_plan(cfg, job.n), counters);
     AFD_CHECK_LAUNCH();
     return AFD_OK;
   };

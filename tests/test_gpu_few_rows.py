@@ -20,7 +20,8 @@ from gpu_util import bits16, dev, rel_l2, say
 from oracle import experts as OX
 from oracle import formats as F
 from sgl_asap_amd import workloads as W
-from sgl_asap_amd.moe.experts import AfdExperts, pack_fp8_block_experts, pack_mxfp4_experts
+from sgl_asap_amd.moe.experts import (AfdExperts, new_job_desc, pack_fp8_block_experts, pack_mxfp4_experts,
+                                      set_job)
 from sgl_asap_amd.moe.topk import StandardTopKOutput
 from test_gpu_moe import deq_weights
 
@@ -130,3 +131,119 @@ def test_concentrated_rows_match_large_tiles(num_local, counts, fmt, act):
     few = call(n)
     assert np.isfinite(F.bf16_to_f32(few)).all()
     assert np.array_equal(few, call(n + more)[:n])
+
+
+# Above 2560 pairs (2048 in groups of 32 rows) a call launches both forms and the router writes its
+# choice: few rows if gate_up's row groups make at most two rounds of workgroups (1024 / image columns
+# groups of 64 rows, 1536 / columns of 32), or there are at most 3/2 groups per expert with rows.
+def spread(experts, rows, last):
+    """``experts`` experts of ``rows`` rows, one more of ``last`` if any."""
+    return [rows] * experts + ([last] if last else [])
+
+
+# num_local, hidden, inter, counts, the router's choice (n: the counts' sum, at least 2700)
+EDGES = [
+    # 16 image columns of gate_up, 80 experts: groups of 64 rows, 64 of them make two rounds
+    (80, 256, 2048, spread(20, 140, 64 * 4), 1),  # 64 groups on 21 experts
+    (80, 256, 2048, spread(20, 140, 64 * 4 + 1), 0),  # 65
+    (80, 256, 2048, spread(25, 65, 0) + spread(25, 50, 0), 1),  # 75 on 50: 3/2
+    (80, 256, 2048, spread(26, 65, 0) + spread(24, 50, 0), 0),  # 76 on 50
+    # 256 experts: groups of 32 rows, 96 of them make two rounds
+    (256, 256, 2048, spread(31, 65, 65), 1),  # 96 groups on 32 experts
+    (256, 256, 2048, spread(31, 65, 97), 0),  # 97
+    (256, 256, 2048, spread(80, 33, 0) + spread(80, 1, 0), 1),  # 240 on 160: 3/2
+    (256, 256, 2048, spread(81, 33, 0) + spread(79, 1, 0), 0),  # 241 on 160
+    (256, 256, 128, [0] * 255 + [4000], 1),  # one column; all rows on the last expert
+]
+
+
+def counted(counts, num_local, total):
+    return (list(counts) + [0] * num_local)[:num_local], max(total, sum(counts))
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block"])
+@pytest.mark.parametrize("edge", range(len(EDGES)))
+def test_router_chooses_at_the_edge(edge, fmt, act):
+    """Either choice gives the bits of the large tiles, on a poisoned workspace, from bf16 and
+    quantized rows, in a batch and from a descriptor with room for more tokens."""
+    num_local, hidden, inter, counts, want = EDGES[edge]
+    counts, n = counted(counts, num_local, 2700)
+    assert FEW_ROWS * num_local >= n > 2560
+    say(f"edge E={num_local} H={hidden} I={inter} {fmt} {act} n={n} want={want}")
+    more = GATED * num_local + 1
+    gen = W.generator("cpu", 31 + edge)
+    x = W.tokens(n + more, hidden, gen, "cpu").to(dev())
+    w = (torch.rand(n + more, 1, generator=gen) + 0.25).to(dev())
+    ids = torch.cat([ids_for(counts, num_local, n, gen),
+                     torch.randint(0, num_local, (more, 1), generator=gen, dtype=torch.int32)]).to(dev())
+    gpu = torch.Generator(device=dev()).manual_seed(7)
+    w13 = torch.randn(num_local, 2 * inter, hidden, generator=gpu, device=dev()) * 0.05
+    w2 = torch.randn(num_local, hidden, inter, generator=gpu, device=dev()) * 0.05
+    pack = pack_mxfp4_experts if fmt == "mxfp4" else pack_fp8_block_experts
+    experts = AfdExperts(num_local + 1, 1, 0, range(num_local), pack(w13, w2), n_max=n + more,
+                         act_format="bf16" if act == "bf16" else None)
+
+    def topk(a, b):
+        return StandardTopKOutput(w[a:b].contiguous(), ids[a:b].contiguous())
+
+    def poisoned():
+        experts.workspace().fill_(0xFF)
+        out = torch.empty(n, hidden, dtype=torch.bfloat16, device=dev())
+        out.view(torch.int16).fill_(-1)
+        return out
+
+    def chosen():
+        return int(experts.ws_view("num_tiles", torch.int32, 2, n)[1])
+
+    ref = bits16(experts(x, topk(0, n + more)))[:n]  # the large tiles
+    assert np.isfinite(F.bf16_to_f32(ref)).all()
+    got = bits16(experts(x[:n].contiguous(), topk(0, n), out=poisoned()))
+    assert chosen() == want
+    assert np.array_equal(got, ref)
+    if act == "fp8":
+        xq, xs = experts.quant_act(x[:n].contiguous())
+        got = bits16(experts.forward_q(xq, xs, topk(0, n), out=poisoned()))
+        assert chosen() == want
+        assert np.array_equal(got, ref)
+    cut, out = n // 3, poisoned()
+    experts.forward_batch([(x[:cut].contiguous(), topk(0, cut)), (x[cut:n].contiguous(), topk(cut, n))],
+                          outs=[out[:cut], out[cut:]])
+    torch.cuda.synchronize()
+    assert chosen() == want
+    assert np.array_equal(bits16(out), ref)
+    if n + 8 <= FEW_ROWS * num_local:  # room for more tokens, in the same form
+        desc, out, job = new_job_desc(dev()), poisoned(), topk(0, n)
+        set_job(desc, ids=job.topk_ids, w=job.topk_weights, out=out, x=x[:n].contiguous())
+        experts.call_job(desc, n + 8)
+        torch.cuda.synchronize()
+        assert int(experts.ws_view("num_tiles", torch.int32, 2, n + 8)[1]) == want
+        assert np.array_equal(bits16(out), ref)
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("extra,want", [(0, 1), (1, 0)])
+def test_local_pairs_at_the_line(extra, want, act):
+    """An MXFP4 call above the few-rows line: local pairs exactly at 40 per local expert, and one
+    more."""
+    num_local, hidden, inter = 42, 256, 128
+    counts = spread(num_local - 1, FEW_ROWS, FEW_ROWS + extra)
+    n, more = FEW_ROWS * num_local + 301, GATED * num_local + 1
+    gen = W.generator("cpu", 41)
+    x = W.tokens(n + more, hidden, gen, "cpu")
+    w = torch.rand(n + more, 1, generator=gen) + 0.25
+    ids = torch.cat([ids_for(counts, num_local, n, gen),
+                     torch.randint(0, num_local, (more, 1), generator=gen, dtype=torch.int32)])
+    w13, w2 = W.expert_weights(num_local, hidden, inter, gen, "cpu")
+    experts = AfdExperts(4 * num_local, 1, 0, range(num_local), pack_mxfp4_experts(w13, w2, device=dev()),
+                         n_max=n + more, act_format="bf16" if act == "bf16" else None)
+
+    def call(m):
+        experts.workspace().fill_(0xFF)
+        out = experts(x[:m].to(dev()), StandardTopKOutput(w[:m].to(dev()), ids[:m].to(dev())))
+        torch.cuda.synchronize()
+        return bits16(out)
+
+    got = call(n)
+    assert int(experts.ws_view("num_tiles", torch.int32, 2, n)[1]) == want
+    assert np.array_equal(got, call(n + more)[:n])

@@ -1,0 +1,93 @@
+"""CPU: which GEMMs an expert call runs (afd_rows_rule.h, compiled here as host code).
+
+The few-rows GEMMs read an expert's weights once per group of 64 (or 32) rows, so with the pairs
+concentrated on few experts they lose to the large tiles, on 256 experts by up to 2.2 times. A call
+launches them alone only while it is too small for that; a larger one launches both forms and the
+router's counts choose."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+LARGE, FEW, BOTH = 0, 1, 2
+MXFP4, FP8_BLOCK = 1, 2
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc is not available to build the host program")
+    exe = tmp_path_factory.mktemp("rows_rule") / "rows_rule"
+    subprocess.run([HIPCC, "-O1", "-std=c++17", "-x", "hip", "--cuda-host-only", os.path.join(HERE, "rows_rule.cpp"),
+                    "-o", str(exe)], check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+
+    def run(cases):
+        """cases: dicts; returns (form, group rows, the router's choice) of each. ``counts``: rows per expert."""
+        lines = []
+        for c in cases:
+            n, k, local = c["n"], c.get("topk", 8), c["local"]
+            rows = 32 if n * k <= 16 * local else 64
+            counts = c.get("counts", [])
+            lines.append(f"{c['fmt']} {c.get('inter', 2048)} {k} {c.get('lo', 0)} {local} {c.get('walk', 0)} {n} "
+                         f"{sum(counts)} {sum(-(-v // rows) for v in counts)} {sum(v > 0 for v in counts)}")
+        res = subprocess.run([str(exe)], input="\n".join(lines) + "\n", stdout=subprocess.PIPE, text=True, timeout=60,
+                             check=True)
+        return [tuple(int(v) for v in line.split()) for line in res.stdout.splitlines()]
+
+    return run
+
+
+@pytest.mark.parametrize("fmt", [MXFP4, FP8_BLOCK])
+def test_form_and_group_rows_at_the_lines(rule, fmt):
+    cases = [
+        (dict(local=64, n=1), (FEW, 32)),
+        (dict(local=64, n=128), (FEW, 32)),  # 16 pairs per expert
+        (dict(local=64, n=129), (FEW, 64)),
+        (dict(local=64, n=320), (FEW, 64)),  # 40 pairs per expert, 2560 pairs
+        (dict(local=64, n=321), (BOTH if fmt == MXFP4 else LARGE, 64)),
+        (dict(local=65, n=2560, topk=1), (FEW, 64)),
+        (dict(local=65, n=2561, topk=1), (BOTH, 64)),
+        (dict(local=256, n=256), (FEW, 32)),  # 2048 pairs
+        (dict(local=256, n=257), (BOTH, 32)),
+        (dict(local=256, n=512), (BOTH, 32)),
+        (dict(local=256, n=513), (BOTH, 64)),
+        (dict(local=256, n=1280), (BOTH, 64)),
+        (dict(local=1, n=5), (FEW, 64)),
+        (dict(local=1, n=2, topk=8), (FEW, 32)),
+        (dict(local=64, n=131071), (LARGE, 64)),
+    ]
+    got = rule([dict(c, fmt=fmt) for c, _ in cases])
+    assert [g[:2] for g in got] == [want for _, want in cases]
+
+
+@pytest.mark.parametrize("fmt", [MXFP4, FP8_BLOCK])
+def test_concentrated_routing_takes_the_large_tiles(rule, fmt):
+    """Routings measured: those the few-rows GEMMs lost by 20% and more go to the large tiles, even
+    loads and Zipf-like ones stay with the few rows."""
+    hot = lambda total, m, local: [total // m] * m + [0] * (local - m)
+    large = [dict(local=256, n=1280, counts=hot(10240, m, 256)) for m in (8, 32, 64, 128)]
+    large += [dict(local=256, n=510, counts=hot(4080, m, 256)) for m in (16, 32, 64)]
+    large += [dict(local=128, n=640, counts=hot(5120, m, 128)) for m in (12, 16, 32, 64)]
+    few = [dict(local=256, n=1280, counts=[40] * 256), dict(local=256, n=510, counts=[15] * 256),
+           dict(local=128, n=640, counts=[40] * 128),
+           dict(local=256, n=1280, counts=[700, 300, 200, 100] + [35] * 252)]
+    got = rule([dict(c, fmt=fmt) for c in large + few])
+    assert all(form == BOTH for form, _, _ in got)
+    assert [choice for _, _, choice in got] == [0] * len(large) + [1] * len(few)
+
+
+@pytest.mark.parametrize("local,inter", [(64, 2048), (65, 1536), (128, 2048), (256, 1024), (256, 2048)])
+@pytest.mark.parametrize("fmt", [MXFP4, FP8_BLOCK])
+def test_few_rows_run_alone_only_in_small_calls(rule, fmt, local, inter):
+    sizes = list(range(1, 6 * local))
+    for n, (form, rows, _) in zip(sizes, rule([dict(fmt=fmt, local=local, inter=inter, n=n) for n in sizes])):
+        pairs = 8 * n
+        if pairs > 40 * local:
+            assert form == (BOTH if fmt == MXFP4 and pairs <= 140 * local else LARGE), n
+        else:
+            assert form == (FEW if pairs <= (2048 if rows == 32 else 2560) else BOTH), n
+            assert rows == (32 if pairs <= 16 * local else 64), n
