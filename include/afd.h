@@ -125,6 +125,14 @@ enum afd_tile_walk {
                           counter costs 1-4%) */
 };
 
+/* tile_walk may also say how many experts the model has, in the bits above the walk:
+ * walk | experts << AFD_NUM_EXPERTS_SHIFT, at least expert_lo + num_local (0: not said, the
+ * experts up to this rank's last one). Like the walk it is about time alone: of a call with many
+ * pairs per local expert, an MXFP4 rank that owns a small share of the experts may still have few
+ * local ones, and then launches two forms of the GEMMs for the router's count to choose from. */
+#define AFD_WALK_MASK 0xff
+#define AFD_NUM_EXPERTS_SHIFT 8
+
 /* Shape of one MoE layer on one F rank. Experts [expert_lo, expert_lo + num_local) are
  * local; top-k ids are global expert ids; pairs with other ids are skipped.
  * Limits: hidden a multiple of 256 up to 16384, inter a multiple of 128 up to 16384,
@@ -139,7 +147,7 @@ typedef struct afd_moe_cfg {
   int32_t activation; /* enum afd_activation (0: SwiGLU) */
   float act_alpha;    /* SiTU: A > 0 (unused otherwise) */
   float act_limit;    /* SiTU, SwiGLU with limit: L > 0 and finite (unused for SwiGLU) */
-  int32_t tile_walk;  /* enum afd_tile_walk (0: static) */
+  int32_t tile_walk;  /* enum afd_tile_walk (0: static), | experts << AFD_NUM_EXPERTS_SHIFT */
   int32_t act_fmt;    /* enum afd_act_fmt (0: fp8) */
 } afd_moe_cfg;
 

@@ -705,7 +705,7 @@ int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
   p.rows_desc = rows_desc;
   p.b = static_cast<const uint8_t*>(wt.w13);
   p.bs = static_cast<const float*>(wt.s13);
-  p.walk_ctr = cfg.tile_walk == AFD_WALK_DYNAMIC ? call_counters(ws, L) + kGateUpWalkWord : nullptr;
+  p.walk_ctr = dynamic_walk(cfg) ? call_counters(ws, L) + kGateUpWalkWord : nullptr;
   p.K = cfg.hidden;
   p.N = 2 * cfg.inter;
   p.hq = ws + L.hq;
@@ -721,7 +721,7 @@ int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_
   p.as = reinterpret_cast<const float*>(ws + L.hs);
   p.b = static_cast<const uint8_t*>(wt.w2);
   p.bs = static_cast<const float*>(wt.s2);
-  p.walk_ctr = cfg.tile_walk == AFD_WALK_DYNAMIC ? call_counters(ws, L) + kDownWalkWord : nullptr;
+  p.walk_ctr = dynamic_walk(cfg) ? call_counters(ws, L) + kDownWalkWord : nullptr;
   p.K = cfg.inter;
   p.N = cfg.hidden;
   p.y = reinterpret_cast<uint16_t*>(ws + L.y);

@@ -695,7 +695,7 @@ int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint
   p.num_tiles = reinterpret_cast<const int32_t*>(ws + L.num_tiles);
   p.padded_offsets = reinterpret_cast<const int32_t*>(ws + L.padded_offsets);
   p.counts = reinterpret_cast<const int32_t*>(ws + L.counts);
-  p.walk_ctr = cfg.tile_walk == AFD_WALK_DYNAMIC ? call_counters(ws, L) + kGateUpWalkWord : nullptr;
+  p.walk_ctr = dynamic_walk(cfg) ? call_counters(ws, L) + kGateUpWalkWord : nullptr;
   p.K = cfg.hidden;
   p.N = 2 * cfg.inter;
   p.h_img = ws + L.hq;
@@ -721,7 +721,7 @@ int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t
   p.num_tiles = reinterpret_cast<const int32_t*>(ws + L.num_tiles);
   p.padded_offsets = reinterpret_cast<const int32_t*>(ws + L.padded_offsets);
   p.counts = reinterpret_cast<const int32_t*>(ws + L.counts);
-  p.walk_ctr = cfg.tile_walk == AFD_WALK_DYNAMIC ? call_counters(ws, L) + kDownWalkWord : nullptr;
+  p.walk_ctr = dynamic_walk(cfg) ? call_counters(ws, L) + kDownWalkWord : nullptr;
   p.K = cfg.inter;
   p.N = cfg.hidden;
   p.h_img = nullptr;

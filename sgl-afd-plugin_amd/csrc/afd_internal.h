@@ -21,7 +21,9 @@ inline int block_m_of(const afd_moe_cfg& cfg) {
   return cfg.weight_fmt == AFD_W_FP8_BLOCK && cfg.act_fmt == AFD_A_FP8 ? kFp8BlockM : kBlockM;
 }
 constexpr int kMaxBatch = AFD_MAX_BATCH;  // jobs of one batched call
-
+inline bool dynamic_walk(const afd_moe_cfg& cfg) {
+  return (cfg.tile_walk & AFD_WALK_MASK) == AFD_WALK_DYNAMIC;
+}
 
 // Where a launch finds its job: the fields by value, or (desc != nullptr) read from the job
 // descriptor in device memory when the kernel runs, its n then clamped to [0, n], n being

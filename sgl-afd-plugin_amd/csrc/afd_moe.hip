@@ -271,7 +271,9 @@ static int check_cfg(const afd_moe_cfg* cfg) {
     return AFD_ERR_ARG;
   if (cfg->activation == AFD_ACT_SWIGLU_LIMIT && !(cfg->act_limit > 0.0f && cfg->act_limit < INFINITY))
     return AFD_ERR_ARG;
-  if (cfg->tile_walk != AFD_WALK_STATIC && cfg->tile_walk != AFD_WALK_DYNAMIC) return AFD_ERR_ARG;
+  const int32_t walk = cfg->tile_walk & AFD_WALK_MASK, experts = cfg->tile_walk >> AFD_NUM_EXPERTS_SHIFT;
+  if (walk != AFD_WALK_STATIC && walk != AFD_WALK_DYNAMIC) return AFD_ERR_ARG;
+  if (experts != 0 && experts < int64_t(cfg->expert_lo) + cfg->num_local) return AFD_ERR_ARG;
   if (cfg->act_fmt != AFD_A_FP8 && cfg->act_fmt != AFD_A_BF16) return AFD_ERR_UNSUPPORTED;
   return AFD_OK;
 }

@@ -18,15 +18,17 @@ namespace afd {
 // 236 -> 222 (Zipf 1.2), at 48 210 -> 225 and 245 -> 259, with bf16 activations at 35 366 -> 270.
 constexpr int kFewRowsPerExpert = 40;
 // A call knows its own pairs, not how many of them are local: with at most 40 pairs per local
-// expert if all were, the few-rows GEMMs run. An MXFP4 rank that owns a quarter of
-// a model's experts has the line at four times as many tokens, so nearly up to there both forms
-// are launched and the router's count of local pairs decides between them: 64 of 256 experts, 512
-// tokens 233 -> 185 us, 750 tokens 237 -> 207 (Zipf 1.2), 194 -> 179 (uniform), with bf16
-// activations 512 tokens 334 -> 219, 1024 362 -> 274. Where the large tiles then run after all, the
-// two launches that return at once cost 2 to 5 us (2% at 1200 tokens), which is why this ends a
-// little before a quarter. FP8 experts gain nothing there (32 of 128 experts, 512 tokens: 68 -> 74
-// us) and take the large tiles.
-constexpr int kGatedRowsPerExpert = 140;
+// expert if all were, the few-rows GEMMs run. An MXFP4 rank that owns a quarter of a model's experts
+// has the line at four times as many tokens, so nearly up to there, 35 expected pairs per local
+// expert, both forms are launched and the router's count of local pairs decides between them: 64 of
+// 256 experts, 512 tokens 233 -> 185 us, 750 tokens 237 -> 207 (Zipf 1.2), 194 -> 179 (uniform), with
+// bf16 activations 512 tokens 334 -> 219, 1024 362 -> 274. Where the large tiles then run after all,
+// the two launches that return at once cost 2 to 5 us (2% at 1200 tokens), which is why this ends a
+// little before 40; and a rank that owns all experts, which would always pay them (64 of 64, 560
+// tokens 209 -> 215 us; 32 of 32 of hidden 2048, 800 tokens 101 -> 105), never launches both for
+// this. Measured up to a quarter, hence the second bound. FP8 experts gain nothing there (32 of 128
+// experts, 512 tokens: 68 -> 74 us) and take the large tiles.
+constexpr int kGatedRowsPerModelExpert = 35, kGatedRowsPerExpert = 140;
 // Groups of 32 rows run three workgroups a CU instead of two, groups of 64 read the weights of an
 // expert of 33 to 64 rows once: 32 while few experts have more rows. At most 16 pairs per expert:
 // -6 to +0.6% over the four formats and two routings (64 FP8 experts, bf16 activations, 8 tokens
@@ -63,6 +65,12 @@ struct RowsPlan {
   int32_t max_groups;
 };
 
+// The model's experts, as far as the configuration says: at least those up to this rank's last one.
+inline int64_t model_experts(const afd_moe_cfg& cfg) {
+  const int64_t said = cfg.tile_walk >> AFD_NUM_EXPERTS_SHIFT, seen = int64_t(cfg.expert_lo) + cfg.num_local;
+  return said > seen ? said : seen;
+}
+
 inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n) {
   const int64_t pairs = n * cfg.topk, local = cfg.num_local;
   RowsPlan p;
@@ -73,7 +81,10 @@ inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n) {
   if (pairs <= kFewRowsPerExpert * local)
     p.form = pairs <= (narrow ? kFewPairsNarrow : kFewPairs) ? kRowsFew : kRowsBoth;
   else
-    p.form = cfg.weight_fmt == AFD_W_MXFP4 && pairs <= kGatedRowsPerExpert * local ? kRowsBoth : kRowsLarge;
+    p.form = cfg.weight_fmt == AFD_W_MXFP4 && pairs <= kGatedRowsPerExpert * local &&
+                     pairs <= kGatedRowsPerModelExpert * model_experts(cfg)
+                 ? kRowsBoth
+                 : kRowsLarge;
   return p;
 }
 

@@ -34,6 +34,8 @@ AFD_ACT_SWIGLU_LIMIT = 2
 AFD_WAIT_GEQ, AFD_WAIT_EQ, AFD_WAIT_AND, AFD_WAIT_NOR = 0, 1, 2, 3
 
 AFD_WALK_STATIC, AFD_WALK_DYNAMIC = 0, 1
+# tile_walk also carries the model's number of experts (0: not said)
+AFD_WALK_MASK, AFD_NUM_EXPERTS_SHIFT = 0xFF, 8
 
 # afd_abi_version() of the library these structures match
 ABI_VERSION = 6

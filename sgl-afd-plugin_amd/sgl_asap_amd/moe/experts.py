@@ -183,6 +183,7 @@ def moe_cfg(
     gemm1_alpha: Optional[float] = None,
     gemm1_clamp_limit: Optional[float] = None,
     act_format: Optional[str] = None,
+    num_experts: int = 0,
 ) -> _lib.AfdMoeCfg:
     """The C config of a layer. ``activation`` is FusedMoE's ("silu": SwiGLU; "situ": SiTU
     with ``gemm1_alpha`` = its beta and ``gemm1_clamp_limit`` = its linear_beta, as the
@@ -192,7 +193,8 @@ def moe_cfg(
     precision of the GEMMs' activations, the weight format's fp8 form by default ("mxfp8" for
     MXFP4, "fp8_1x128" for FP8 blocks, the MoE methods' default quantization) or "bf16" (W4A16
     for MXFP4 weights: the reference's humming experts, scripts/run_ep.sh:4, README.md:25;
-    W8A16 for FP8 blocks)."""
+    W8A16 for FP8 blocks). ``num_experts``: the model's experts (0: not said), by which the call
+    expects how many of its pairs are local."""
     fp8 = FP8_ACT[weights.fmt]
     if act_format not in (None, fp8, "bf16"):
         raise ValueError(f"activation format {act_format!r} for {weights.fmt} weights "
@@ -218,10 +220,12 @@ def moe_cfg(
             raise ValueError(f"SiTU constants must be positive and finite, got {alpha}, {limit}")
     return _lib.AfdMoeCfg(
         weights.hidden, weights.inter, top_k, expert_lo, weights.num_local, WEIGHT_FORMATS[weights.fmt],
-        code, alpha, limit, _lib.AFD_WALK_STATIC, act_fmt,
+        code, alpha, limit, _lib.AFD_WALK_STATIC | min(num_experts, MAX_SAID_EXPERTS) << _lib.AFD_NUM_EXPERTS_SHIFT,
+        act_fmt,
     )
 
 
+MAX_SAID_EXPERTS = (1 << 31 - _lib.AFD_NUM_EXPERTS_SHIFT) - 1
 TILE_WALKS = {"static": _lib.AFD_WALK_STATIC, "dynamic": _lib.AFD_WALK_DYNAMIC}
 
 # activation formats of the expert call's input -> the weight format whose GEMMs read them
@@ -384,7 +388,8 @@ class AfdExperts(torch.nn.Module):
         self.weights = weights
         self.n_max = n_max
         self.activation = activation
-        self.cfg = moe_cfg(weights, top_k, local.start, activation, gemm1_alpha, gemm1_clamp_limit, act_format)
+        self.cfg = moe_cfg(weights, top_k, local.start, activation, gemm1_alpha, gemm1_clamp_limit, act_format,
+                           num_experts)
         self.tile_walk = tile_walk
         self.layout = workspace_layout(self.cfg, n_max)
         self._batch_bytes = {n_max: self.layout["total"]}  # workspace bytes per batch capacity
@@ -392,13 +397,14 @@ class AfdExperts(torch.nn.Module):
 
     @property
     def tile_walk(self) -> str:
-        return "dynamic" if self.cfg.tile_walk == _lib.AFD_WALK_DYNAMIC else "static"
+        walk = self.cfg.tile_walk & _lib.AFD_WALK_MASK
+        return "dynamic" if walk == _lib.AFD_WALK_DYNAMIC else "static"
 
     @tile_walk.setter
     def tile_walk(self, walk: str) -> None:
         if walk not in TILE_WALKS:
             raise ValueError(f"tile_walk must be one of {sorted(TILE_WALKS)}, got {walk!r}")
-        self.cfg.tile_walk = TILE_WALKS[walk]
+        self.cfg.tile_walk = self.cfg.tile_walk & ~_lib.AFD_WALK_MASK | TILE_WALKS[walk]
 
     def workspace(self, stream: Optional[torch.cuda.Stream] = None) -> torch.Tensor:
         """The workspace of this layer's calls on ``stream`` (default: current): one per stream

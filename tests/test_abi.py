@@ -185,3 +185,35 @@ def test_python_activation_arguments():
     for bad in (0.0, -1.0, float("inf")):
         with pytest.raises(ValueError):
             moe_cfg(wts, 2, 0, "silu", None, bad)
+
+
+def test_tile_walk_carries_the_experts_of_the_model():
+    """tile_walk: a walk, or a walk and at least as many experts as the configuration shows."""
+    L, out = _lib.lib(), _lib.AfdWsLayout()
+
+    def status(walk, lo=0, local=64):
+        cfg = _lib.AfdMoeCfg(4096, 2048, 8, lo, local, _lib.AFD_W_MXFP4, 0, 0.0, 0.0, walk)
+        return L.afd_workspace_layout(ctypes.byref(cfg), 16, ctypes.byref(out))
+
+    for walk in (0, 1, 64 << 8, 64 << 8 | 1, 256 << 8, (1 << 23) - 1 << 8):
+        assert status(walk) == _lib.AFD_OK, walk
+    assert status(256 << 8, lo=192) == _lib.AFD_OK
+    for walk in (2, 255, 63 << 8, 1 << 8, 64 << 8 | 2, -1, -256, -2**31):
+        assert status(walk) == _lib.AFD_ERR_ARG, walk
+    assert status(255 << 8, lo=192) == _lib.AFD_ERR_ARG
+    assert status(256 << 8, lo=2**31 - 1) == _lib.AFD_ERR_ARG
+    assert status(0, lo=2**31 - 1) == _lib.AFD_OK
+
+
+def test_layer_config_says_the_experts_and_keeps_them_with_the_walk():
+    from sgl_asap_amd.moe.experts import AfdExperts, ExpertWeights, moe_cfg
+
+    import torch
+
+    wts = ExpertWeights("mxfp4", 64, 256, 128, *(torch.empty(0, dtype=torch.uint8) for _ in range(4)))
+    assert moe_cfg(wts, 8, 0).tile_walk == _lib.AFD_WALK_STATIC
+    assert moe_cfg(wts, 8, 0, num_experts=2**40).tile_walk == (2**23 - 1) << 8
+    layer = AfdExperts(256, 8, 0, range(64, 128), wts, n_max=16, tile_walk="dynamic")
+    assert layer.cfg.tile_walk == 256 << 8 | _lib.AFD_WALK_DYNAMIC and layer.tile_walk == "dynamic"
+    layer.tile_walk = "static"
+    assert layer.cfg.tile_walk == 256 << 8 and layer.tile_walk == "static"

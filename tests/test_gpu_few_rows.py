@@ -4,8 +4,9 @@ format, at the sizes where they can go wrong: expert counts around the 32-row bl
 with no row, one K stage and K stages that do not fill the register ring, one and several weight
 image columns, and an expert count that is not a multiple of the 4 a lane looks up.
 
-Above that, up to GATED tokens per local expert, an MXFP4 call launches both the few-rows and
-the large-tile GEMMs and the number of local pairs decides on the GPU; both outcomes are run.
+Above that, up to GATED tokens per local expert on a rank with a quarter of the experts, an MXFP4
+call launches both the few-rows and the large-tile GEMMs and the number of local pairs decides on
+the GPU; both outcomes are run. So does any call above 2560 pairs, by how the pairs are spread.
 
 The large-tile GEMMs and the few-rows GEMMs feed every accumulator the same products in the
 same order, so the same tokens inside a call large enough for the large tiles must give the
@@ -79,7 +80,8 @@ def test_few_rows_match_large_tiles(num_local, hidden, inter, activation, fmt, a
         oact = dict(activation="situ", act_alpha=2.0, act_limit=3.0)
     elif activation == "silu_limit":
         kw, oact = dict(swiglu_limit=0.5), dict(activation="swiglu_limit", act_limit=0.5)
-    experts = AfdExperts(num_local + 1, 1, 0, range(num_local), pack(w13, w2, device=dev()), n_max=n + more,
+    # a rank with a quarter of the experts: more tokens launch both forms
+    experts = AfdExperts(4 * num_local, 1, 0, range(num_local), pack(w13, w2, device=dev()), n_max=n + more,
                          act_format="bf16" if act == "bf16" else None, **kw)
 
     def call(m):

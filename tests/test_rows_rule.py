@@ -48,7 +48,7 @@ def test_form_and_group_rows_at_the_lines(rule, fmt):
         (dict(local=64, n=128), (FEW, 32)),  # 16 pairs per expert
         (dict(local=64, n=129), (FEW, 64)),
         (dict(local=64, n=320), (FEW, 64)),  # 40 pairs per expert, 2560 pairs
-        (dict(local=64, n=321), (BOTH if fmt == MXFP4 else LARGE, 64)),
+        (dict(local=64, n=321, walk=256 << 8), (BOTH if fmt == MXFP4 else LARGE, 64)),
         (dict(local=65, n=2560, topk=1), (FEW, 64)),
         (dict(local=65, n=2561, topk=1), (BOTH, 64)),
         (dict(local=256, n=256), (FEW, 32)),  # 2048 pairs
@@ -84,10 +84,29 @@ def test_concentrated_routing_takes_the_large_tiles(rule, fmt):
 @pytest.mark.parametrize("fmt", [MXFP4, FP8_BLOCK])
 def test_few_rows_run_alone_only_in_small_calls(rule, fmt, local, inter):
     sizes = list(range(1, 6 * local))
-    for n, (form, rows, _) in zip(sizes, rule([dict(fmt=fmt, local=local, inter=inter, n=n) for n in sizes])):
+    cases = [dict(fmt=fmt, local=local, inter=inter, n=n, walk=4 * local << 8 | n % 2) for n in sizes]
+    for n, (form, rows, _) in zip(sizes, rule(cases)):
         pairs = 8 * n
         if pairs > 40 * local:
             assert form == (BOTH if fmt == MXFP4 and pairs <= 140 * local else LARGE), n
         else:
             assert form == (FEW if pairs <= (2048 if rows == 32 else 2560) else BOTH), n
             assert rows == (32 if pairs <= 16 * local else 64), n
+
+
+@pytest.mark.parametrize("lo,said,last", [
+    (0, 0, 320),  # 64 experts, as far as the configuration says: all local
+    (0, 64, 320),  # all local
+    (0, 65, 320), (0, 80, 350),  # the few-rows line itself; 35 pairs per expert of the model
+    (0, 128, 560), (64, 0, 560), (64, 128, 560),  # half
+    (0, 256, 1120), (192, 0, 1120), (64, 256, 1120),  # a quarter
+    (0, 512, 1120), (448, 0, 1120),  # an eighth: measured up to a quarter
+])
+def test_both_forms_are_launched_only_near_the_line(rule, lo, said, last):
+    """An MXFP4 rank launches both forms for the count of local pairs only where its share of the
+    experts makes few local pairs likely: with all experts local it never does."""
+    sizes = range(1, 1500)
+    got = rule([dict(fmt=MXFP4, local=64, lo=lo, n=n, walk=said << 8 | n % 2) for n in sizes])
+    assert [form for form, _, _ in got] == [FEW if n <= 320 else BOTH if n <= last else LARGE for n in sizes]
+    got = rule([dict(fmt=FP8_BLOCK, local=64, lo=lo, n=n, walk=said << 8 | n % 2) for n in sizes])
+    assert [form for form, _, _ in got] == [FEW if n <= 320 else LARGE for n in sizes]
