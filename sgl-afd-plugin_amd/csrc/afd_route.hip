@@ -27,7 +27,8 @@ namespace afd {
 constexpr int kRouteThreads = 256;
 constexpr int kMaxChunks = 128;
 constexpr int kFusedPairs = 4096;  // up to as many pairs are routed in one launch
-constexpr int kFusedGroups = 16;   // by at least as many workgroups (they share the -1 fill)
+constexpr int kFusedGroups = 16;   // by as many workgroups: those past the last chunk share the -1 fill
+static_assert(kFusedPairs <= kFusedGroups * kRouteThreads, "a workgroup for each chunk of 256 pairs");
 constexpr int kKeyBits = 9;  // keys 0..256 (local expert, or num_local for "not local")
 static_assert(kRouteThreads == kQuantThreads, "the prep kernel's workgroups do either job");
 
@@ -322,11 +323,10 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
     return AFD_OK;
   };
   if (pairs <= kFusedPairs) {
-    const int route_groups = chunks > kFusedGroups ? chunks : kFusedGroups;
-    const int grid = route_groups + quant_grid;
-    const int st = fmt == kPrepMxfp8 ? scatter(route_scatter_kernel<true, kPrepMxfp8>, route_groups, grid)
-                   : fmt == kPrepFp8 ? scatter(route_scatter_kernel<true, kPrepFp8>, route_groups, grid)
-                                     : scatter(route_scatter_kernel<true, kPrepNone>, route_groups, grid);
+    const int grid = kFusedGroups + quant_grid;
+    const int st = fmt == kPrepMxfp8 ? scatter(route_scatter_kernel<true, kPrepMxfp8>, kFusedGroups, grid)
+                   : fmt == kPrepFp8 ? scatter(route_scatter_kernel<true, kPrepFp8>, kFusedGroups, grid)
+                                     : scatter(route_scatter_kernel<true, kPrepNone>, kFusedGroups, grid);
     if (st == AFD_OK && mid) AFD_CHECK_HIP(hipEventRecord(mid, stream));
     return st;
   }

@@ -76,6 +76,24 @@ CASES = [
 ]
 
 
+# up to 4096 pairs are routed in one launch, by 16 workgroups of 256 pairs: at and around the line,
+# with one, a quarter and all experts local
+ONE_LAUNCH = [
+    (n, k, num_experts, e_lo, num_local, 20 + n)
+    for n, k in ((512, 8), (4096, 1), (4097, 1), (4095, 1), (455, 9), (3841, 1), (241, 17))
+    for num_experts, e_lo, num_local in ((64, 7, 1), (256, 64, 64), (256, 0, 256))
+]
+
+
+@pytest.mark.parametrize("fmt", [_lib.AFD_W_MXFP4, _lib.AFD_W_FP8_BLOCK])
+@pytest.mark.parametrize("n,k,num_experts,e_lo,num_local,seed", ONE_LAUNCH)
+def test_route_around_the_one_launch_line(n, k, num_experts, e_lo, num_local, seed, fmt):
+    say(f"route fmt={fmt} n={n} k={k} experts={num_experts} local=[{e_lo},{e_lo + num_local})")
+    g = torch.Generator().manual_seed(seed)
+    ids = torch.topk(torch.rand(n, num_experts, generator=g), k, dim=1).indices.to(torch.int32).numpy()
+    check(ids, e_lo, num_local, fmt)
+
+
 @pytest.mark.parametrize("n,k,num_experts,e_lo,num_local,seed", CASES)
 def test_route_random(n, k, num_experts, e_lo, num_local, seed):
     say(f"route n={n} k={k} experts={num_experts} local=[{e_lo},{e_lo + num_local}) seed={seed}")
