@@ -148,11 +148,13 @@ def test_a16_differs_from_fp8_activations(fmt):
     "hidden,inter,num_experts,e_lo,num_local,k,n,seed",
     [
         (512, 256, 32, 8, 16, 4, 300, 1),      # down N = 512: 512-column tiles; gate_up N = 512
-        (256, 128, 16, 0, 16, 8, 1, 2),        # one token; 256-column tiles in both GEMMs
+        (256, 128, 16, 0, 16, 8, 1, 2),        # one token: the few-rows GEMMs
         (1024, 512, 64, 16, 16, 6, 513, 3),
         (2048, 1024, 32, 0, 8, 8, 256, 4),
         (4096, 512, 256, 0, 4, 8, 64, 10),
-        (768, 384, 16, 0, 16, 2, 129, 5),      # down N = 768 (256-column tiles), K stages 6 / 3
+        (768, 384, 16, 0, 16, 2, 129, 5),      # the few-rows GEMMs, K stages 6 / 3
+        (768, 384, 16, 0, 16, 8, 129, 6),      # the same as large tiles: down N = 768, 256-column tiles
+        (256, 128, 8, 0, 8, 8, 41, 7),         # 256-column tiles in both GEMMs
     ],
 )
 def test_a16_layers(hidden, inter, num_experts, e_lo, num_local, k, n, seed):
@@ -164,9 +166,11 @@ def test_a16_layers(hidden, inter, num_experts, e_lo, num_local, k, n, seed):
     "hidden,inter,num_experts,e_lo,num_local,k,n,seed,zipf",
     [
         (512, 256, 32, 8, 16, 4, 300, 51, None),     # 512-column tiles in both GEMMs
-        (256, 128, 16, 0, 16, 8, 1, 52, None),       # one token; 256-column tiles
+        (256, 128, 16, 0, 16, 8, 1, 52, None),       # one token: the few-rows GEMMs
         (1024, 384, 16, 0, 16, 8, 700, 53, 1.1),     # K blocks 8 / 3, down N = 1024
-        (768, 640, 8, 0, 8, 2, 129, 54, None),       # down N = 768: 256-column tiles; 10 K stages
+        (768, 640, 8, 0, 8, 2, 129, 54, None),       # the few-rows GEMMs, K stages 6 / 5
+        (768, 640, 8, 0, 8, 4, 129, 56, None),       # large tiles: down N = 768, 256 columns; 10 K stages
+        (256, 128, 8, 0, 8, 8, 41, 57, None),        # 256-column tiles in both GEMMs
         (4096, 1536, 64, 0, 4, 8, 96, 55, None),     # the ERNIE-style shape on 4 experts
     ],
 )
@@ -204,9 +208,10 @@ def draw(case: int) -> dict:
 
 @pytest.mark.parametrize("case", range(24))
 def test_a16_random_layer(case):
-    """Seeded random shapes: both weight formats, hidden 256-1536, inter 128-768 (both tile
-    widths, 1-12 K stages), token counts around the 128-row tile edge, partial local ranges,
-    top-1 to top-8, uniform and Zipf routing, the three activations, both tile walks."""
+    """Seeded random shapes: both weight formats, hidden 256-1536, inter 128-768 (1-12 K stages),
+    token counts around the 128-row tile edge, partial local ranges, top-1 to top-8, uniform and
+    Zipf routing, the three activations, both tile walks. Two in three run the few-rows GEMMs; the
+    large tiles' small calls are drawn in test_gpu_sweep."""
     s = draw(case)
     extra = {k: s[k] for k in ("situ", "swiglu_limit") if k in s}
     experts, out, ref, parts, (x, ids, w) = run_case(

@@ -1,8 +1,10 @@
 """GPU: seeded random layer shapes against the oracle, across both weight formats and the
 three activations, with token counts at and around the 128-row tile edge (1, 2, 127, 128,
-129, ...), partial local expert ranges and top-k from 1 to 8; and shapes of 2048-4096 tokens
-where every GEMM workgroup takes several tiles, with both tile walks and bf16 activations.
-Same bars as test_gpu_moe."""
+129, ...), partial local expert ranges and top-k from 1 to 8 (up to 40 pairs per local expert these
+run the few-rows GEMMs, the others the large tiles); small shapes above that line, where the rows of
+an expert stand around the 128- and 256-row tile edges, with both tile walks and bf16 activations; and
+shapes of 2048-4096 tokens where every GEMM workgroup takes several tiles. Same bars as
+test_gpu_moe."""
 
 import random
 
@@ -46,6 +48,42 @@ def test_random_layer(case):
     experts, out, ref, parts, (x, ids, w) = run_case(
         s["hidden"], s["inter"], s["num_experts"], s["e_lo"], s["num_local"], s["k"], s["n"], s["fmt"],
         9000 + case, zipf=s["zipf"], **extra)
+    assert_close(out, ref, ids.numpy(), range(s["e_lo"], s["e_lo"] + s["num_local"]))
+
+
+def draw_few_tiles(case: int) -> dict:
+    """Small calls of the large-tile GEMMs: 1 to 6 local experts with more than 140 pairs each (the
+    few-rows GEMMs end at 140 at the latest), tokens at the tile edges, both walks, bf16 and fp8
+    activations, three activations."""
+    rng = random.Random(7700 + case)
+    num_experts = rng.choice([4, 6, 8])
+    num_local = rng.randint(1, 6 if num_experts == 8 else num_experts)
+    k = rng.randint(2, num_experts)
+    least = 140 * num_local // k + 1
+    return dict(
+        fmt=rng.choice(["mxfp4", "fp8_block"]),
+        hidden=256 * rng.randint(1, 6),
+        inter=128 * rng.randint(1, 6),
+        num_experts=num_experts,
+        num_local=num_local,
+        e_lo=rng.randint(0, num_experts - num_local),
+        k=k,
+        n=max(least, rng.choice([least, 127, 128, 129, 255, 256, 257, 400])),
+        zipf=rng.choice([None, 1.2]),
+        walk=rng.choice(["static", "dynamic"]),
+        act_format=rng.choice([None, "bf16"]),
+        act=rng.choice(["silu", "situ", "limit"]),
+    )
+
+
+@pytest.mark.parametrize("case", range(CASES))
+def test_random_layer_few_tiles(case):
+    s = draw_few_tiles(case)
+    assert s["n"] * s["k"] > 140 * s["num_local"]
+    extra = {"situ": dict(situ=(1.702, 7.0)), "limit": dict(swiglu_limit=1.0)}.get(s["act"], {})
+    experts, out, ref, parts, (x, ids, w) = run_case(
+        s["hidden"], s["inter"], s["num_experts"], s["e_lo"], s["num_local"], s["k"], s["n"], s["fmt"],
+        9300 + case, zipf=s["zipf"], walk=s["walk"], act_format=s["act_format"], **extra)
     assert_close(out, ref, ids.numpy(), range(s["e_lo"], s["e_lo"] + s["num_local"]))
 
 

@@ -1,10 +1,11 @@
 """GPU: the two tile walks of the persistent GEMMs give identical results. "dynamic" hands
 the tiles out from per-XCD counters, "static" gives each workgroup a fixed share; both run
 over the same dense tile order, so every output bit must agree, for both weight formats with
-fp8 or bf16 activations, for jobs from one token (8 row tiles, fewer than the 32 needed
-to split the rows over the XCDs) to thousands, for skewed routing, and while another stream
+fp8 or bf16 activations, for jobs from 8 row tiles (fewer than the 32 needed to split the rows over
+the XCDs) to thousands of tokens, for skewed routing, and while another stream
 holds a parked wait (a CU held by a wait kernel: the dynamic walk must still cover every
-tile).
+tile). The calls of 1 to 7 tokens on 16 and 32 experts run the few-rows GEMMs, which have no walk:
+there the setting must not matter.
 
 Before every call the whole workspace and the output are filled with 0xFF bytes, a NaN in
 every format the kernels write there (bf16 y and h, e4m3 h, UE8M0 and fp32 scales), and the
@@ -26,6 +27,7 @@ import pytest
 import torch
 
 from gpu_util import bits16, dev, say
+from oracle import formats as F
 from sgl_asap_amd import workloads as W
 from sgl_asap_amd.moe.experts import AfdExperts, pack_fp8_block_experts, pack_mxfp4_experts
 from sgl_asap_amd.moe.topk import StandardTopKOutput
@@ -100,6 +102,41 @@ def test_walks_agree_across_shapes(hidden, inter):
         x, topk = job(n, hidden, 16, seed, zipf)
         s, d = both(experts, x, topk)
         assert np.array_equal(s, d), (hidden, inter, n, seed)
+
+
+@pytest.mark.parametrize("hidden,inter", [(1024, 512), (768, 384), (256, 128)])
+@pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block", "mxfp4_a16", "fp8_block_a16"])
+def test_walks_agree_below_the_split(fmt, hidden, inter):
+    """Fewer than 32 row tiles, so every workgroup walks all of them: 8 experts, each with all n
+    tokens, more than the few-rows GEMMs take."""
+    experts = layer(fmt, hidden, inter, 8, 400, seed=hidden)
+    rows = experts.layout_for(1)["block_m"]
+    for n, seed in ((41, 21), (128, 22), (129, 23), (300, 24)):
+        say(f"walks below the split fmt={fmt} H={hidden} I={inter} n={n}")
+        x, topk = job(n, hidden, 8, seed)
+        s, d = both(experts, x, topk)
+        assert int(experts.ws_view("num_tiles", torch.int32, 1, n)[0]) == 8 * -(-n // rows) < 32
+        assert np.array_equal(s, d), n
+
+
+@pytest.mark.parametrize("act", [None, "bf16"])
+def test_walks_agree_just_above_the_local_line(act):
+    """An MXFP4 call that launches both forms of the GEMMs, with one local pair more than the
+    few-rows ones take: 8 of 32 experts local, 321 local pairs on 8 row tiles."""
+    n, num_local = 140, 8
+    gen = W.generator("cpu", 25)
+    w13, w2 = W.expert_weights(num_local, 1024, 512, gen, "cpu")
+    experts = AfdExperts(32, 8, 0, range(num_local), pack_mxfp4_experts(w13, w2, device=dev()), n_max=n,
+                         act_format=act)
+    x = W.tokens(n, 1024, gen, "cpu").to(dev())
+    ids = torch.arange(8, 16, dtype=torch.int32).repeat(n, 1)  # no local expert
+    ids[10:50] = torch.arange(8, dtype=torch.int32)
+    ids[70, 3] = 5
+    topk = StandardTopKOutput((torch.rand(n, 8, generator=gen) + 0.25).to(dev()), ids.to(dev()))
+    s, d = both(experts, x, topk)
+    assert experts.ws_view("num_tiles", torch.int32, 2, n).tolist() == [8, 0]  # row tiles; the large tiles chosen
+    assert np.array_equal(s, d)
+    assert F.bf16_to_f32(s)[10:50].any(axis=1).all() and not F.bf16_to_f32(s)[50:70].any()
 
 
 def test_dynamic_walk_with_a_parked_wait():
