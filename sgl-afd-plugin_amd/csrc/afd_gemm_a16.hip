@@ -618,9 +618,9 @@ int launch_a16_any(const A16GemmArgs& p, int max_row_tiles, hipStream_t stream) 
   return launch_a16<WF, MODE, 2>(p, max_row_tiles, stream);
 }
 
-A16GemmArgs a16_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
+A16GemmArgs a16_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, const RowsPlan& plan) {
   A16GemmArgs p = {};
-  p.gate = rows_gate(cfg, ws, L, n);
+  p.gate = rows_gate(plan, ws, L);
   p.topk = cfg.topk;
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
@@ -642,8 +642,8 @@ int gate_up(const A16GemmArgs& p, const afd_moe_cfg& cfg, int max_tiles, hipStre
 
 int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint16_t* x, const afd_job* rows_desc,
-                       int32_t n, hipStream_t stream) {
-  A16GemmArgs p = a16_args(cfg, ws, L, n);
+                       const RowsPlan& plan, hipStream_t stream) {
+  A16GemmArgs p = a16_args(cfg, ws, L, plan);
   p.a_rows = x;
   p.rows_desc = rows_desc;
   p.b_img = static_cast<const uint8_t*>(wt.w13);
@@ -657,8 +657,8 @@ int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
 }
 
 int launch_a16_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  A16GemmArgs p = a16_args(cfg, ws, L, n);
+                    const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream) {
+  A16GemmArgs p = a16_args(cfg, ws, L, plan);
   p.a_img = ws + L.hq;
   p.b_img = static_cast<const uint8_t*>(wt.w2);
   p.b_scale = static_cast<const float*>(wt.s2);

@@ -680,9 +680,9 @@ static int launch(const Fp8GemmArgs& p, int max_row_tiles, hipStream_t stream) {
   return AFD_OK;
 }
 
-static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
+static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, const RowsPlan& plan) {
   Fp8GemmArgs p = {};
-  p.gate = rows_gate(cfg, ws, L, n);
+  p.gate = rows_gate(plan, ws, L);
   p.topk = cfg.topk;
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
@@ -698,8 +698,8 @@ static Fp8GemmArgs common_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws
 
 int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                       const afd_job* rows_desc, int32_t n, hipStream_t stream) {
-  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, n);
+                       const afd_job* rows_desc, const RowsPlan& plan, hipStream_t stream) {
+  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, plan);
   p.a = xq;
   p.as = static_cast<const float*>(xs);
   p.rows_desc = rows_desc;
@@ -715,8 +715,8 @@ int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uin
 }
 
 int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, n);
+                    const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream) {
+  fp8::Fp8GemmArgs p = fp8::common_args(cfg, ws, L, plan);
   p.a = ws + L.hq;
   p.as = reinterpret_cast<const float*>(ws + L.hs);
   p.b = static_cast<const uint8_t*>(wt.w2);

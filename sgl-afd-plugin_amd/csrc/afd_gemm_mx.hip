@@ -679,9 +679,9 @@ static int launch_mx_any(const MxGemmArgs& p, int max_row_tiles, hipStream_t str
 
 int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                       const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                      const afd_job* rows_desc, int32_t n, hipStream_t stream) {
+                      const afd_job* rows_desc, const RowsPlan& plan, hipStream_t stream) {
   MxGemmArgs p;
-  p.gate = rows_gate(cfg, ws, L, n);
+  p.gate = rows_gate(plan, ws, L);
   p.a_img = nullptr;
   p.a_rows = xq;
   p.a_scales = static_cast<const uint8_t*>(xs);
@@ -705,9 +705,9 @@ int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint
 }
 
 int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                   const afd_ws_layout& L, int32_t n, hipStream_t stream) {
+                   const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream) {
   MxGemmArgs p;
-  p.gate = rows_gate(cfg, ws, L, n);
+  p.gate = rows_gate(plan, ws, L);
   p.act = act_params(cfg);
   p.a_img = ws + L.hq;
   p.a_rows = nullptr;

@@ -627,13 +627,8 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
 }
 
 template <int FMT, int MODE>
-int launch_rows(const RowsArgs& p, const RowsPlan& plan, int64_t pairs, hipStream_t stream) {
-  const int cols = p.N / kImgBRows;
-  // row groups of so many pairs: at most one per pair, and one per expert plus one per full group
-  // (gated: of at most max_pairs local pairs)
-  if (plan.form == kRowsBoth && pairs > plan.max_pairs) pairs = plan.max_pairs;
-  const int64_t most = p.num_local + (pairs >> plan.group_shift);
-  const dim3 grid(static_cast<unsigned>((pairs < most ? pairs : most) * cols));
+int launch_rows(const RowsArgs& p, const RowsPlan& plan, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(plan.grid_groups * (p.N / kImgBRows)));
   if (plan.group_shift == 5)
     hipLaunchKernelGGL((rows_gemm_kernel<FMT, MODE, 1>), grid, dim3(256), 0, stream, p);
   else
@@ -643,19 +638,17 @@ int launch_rows(const RowsArgs& p, const RowsPlan& plan, int64_t pairs, hipStrea
 }
 
 template <int MODE>
-int launch_fmt(const RowsArgs& p, const afd_moe_cfg& cfg, int32_t n, hipStream_t stream) {
-  const RowsPlan plan = rows_plan(cfg, n);
-  const int64_t pairs = int64_t(n) * cfg.topk;
+int launch_fmt(const RowsArgs& p, const afd_moe_cfg& cfg, const RowsPlan& plan, hipStream_t stream) {
   if (cfg.act_fmt == AFD_A_BF16)
-    return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx16, MODE>(p, plan, pairs, stream)
-                                         : launch_rows<kF16, MODE>(p, plan, pairs, stream);
-  return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx8, MODE>(p, plan, pairs, stream)
-                                       : launch_rows<kF8, MODE>(p, plan, pairs, stream);
+    return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx16, MODE>(p, plan, stream)
+                                         : launch_rows<kF16, MODE>(p, plan, stream);
+  return cfg.weight_fmt == AFD_W_MXFP4 ? launch_rows<kMx8, MODE>(p, plan, stream)
+                                       : launch_rows<kF8, MODE>(p, plan, stream);
 }
 
-RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
+RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, const RowsPlan& plan) {
   RowsArgs p = {};
-  p.gate = rows_gate(cfg, ws, L, n);
+  p.gate = rows_gate(plan, ws, L);
   p.topk_magic = div_magic(cfg.topk);
   p.act = act_params(cfg);
   p.sorted_pairs = reinterpret_cast<const int32_t*>(ws + L.sorted_pairs);
@@ -666,15 +659,15 @@ RowsArgs rows_args(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, 
 
 }  // namespace
 
-RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n) {
-  if (rows_plan(cfg, n).form != kRowsBoth) return RowsGate{nullptr};
+RowsGate rows_gate(const RowsPlan& plan, uint8_t* ws, const afd_ws_layout& L) {
+  if (plan.form != kRowsBoth) return RowsGate{nullptr};
   return RowsGate{reinterpret_cast<const int32_t*>(call_counters(ws, L)) + kRowsFewWord};
 }
 
 int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                         const afd_ws_layout& L, const void* x, const void* xs, const afd_job* rows_desc,
-                        int32_t n, hipStream_t stream) {
-  RowsArgs p = rows_args(cfg, ws, L, n);
+                        const RowsPlan& plan, hipStream_t stream) {
+  RowsArgs p = rows_args(cfg, ws, L, plan);
   p.a = static_cast<const uint8_t*>(x);
   p.as = static_cast<const uint8_t*>(xs);
   p.rows_desc = rows_desc;
@@ -685,13 +678,13 @@ int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, ui
   p.ntn_magic = div_magic(p.N / kImgBRows);
   p.hq = ws + L.hq;
   p.hs = reinterpret_cast<float*>(ws + L.hs);
-  return cfg.activation != AFD_ACT_SWIGLU ? launch_fmt<kGateUpParam>(p, cfg, n, stream)
-                                         : launch_fmt<kGateUp>(p, cfg, n, stream);
+  return cfg.activation != AFD_ACT_SWIGLU ? launch_fmt<kGateUpParam>(p, cfg, plan, stream)
+                                         : launch_fmt<kGateUp>(p, cfg, plan, stream);
 }
 
 int launch_rows_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                     const afd_ws_layout& L, int32_t n, hipStream_t stream) {
-  RowsArgs p = rows_args(cfg, ws, L, n);
+                     const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream) {
+  RowsArgs p = rows_args(cfg, ws, L, plan);
   p.a = ws + L.hq;
   p.as = ws + L.hs;
   p.b = static_cast<const uint8_t*>(wt.w2);
@@ -700,7 +693,7 @@ int launch_rows_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8
   p.N = cfg.hidden;
   p.ntn_magic = div_magic(p.N / kImgBRows);
   p.y = reinterpret_cast<uint16_t*>(ws + L.y);
-  return launch_fmt<kDown>(p, cfg, n, stream);
+  return launch_fmt<kDown>(p, cfg, plan, stream);
 }
 
 }  // namespace afd

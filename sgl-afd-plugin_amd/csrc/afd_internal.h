@@ -128,7 +128,7 @@ int launch_quant_act(const afd_moe_cfg& cfg, const uint16_t* x, int32_t n, uint8
 // is recorded between the two launches (with few pairs there is one, and it follows that).
 // The first launch also zeroes the call's counter words.
 int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, uint8_t* ws,
-                       const afd_ws_layout& L, hipStream_t stream, hipEvent_t mid);
+                       const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream, hipEvent_t mid);
 
 // Grouped MXFP4 GEMMs (afd_gemm_mx.hip).
 // xq / xs: the quantized activation rows [n][H] and their scales (the workspace's, or the
@@ -136,42 +136,42 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
 // descriptor's xq / xs when the kernel runs.
 int launch_mx_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                       const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                      const afd_job* rows_desc, int32_t n, hipStream_t stream);
+                      const afd_job* rows_desc, const RowsPlan& plan, hipStream_t stream);
 int launch_mx_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                   const afd_ws_layout& L, int32_t n, hipStream_t stream);
+                   const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream);
 
 // Grouped MXFP4-weight x bf16-activation GEMMs (afd_gemm_a16.hip). x: the bf16 token rows
 // [n][H] (the job's, or a batch's staged in the workspace); with rows_desc != nullptr they are
 // that job descriptor's x, read when the kernel runs.
 int launch_a16_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint16_t* x, const afd_job* rows_desc,
-                       int32_t n, hipStream_t stream);
+                       const RowsPlan& plan, hipStream_t stream);
 int launch_a16_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, int32_t n, hipStream_t stream);
+                    const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream);
 
 // Grouped FP8 128x128-block GEMMs (afd_gemm_fp8.hip).
 int launch_fp8_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                        const afd_ws_layout& L, const uint8_t* xq, const void* xs,
-                       const afd_job* rows_desc, int32_t n, hipStream_t stream);
+                       const afd_job* rows_desc, const RowsPlan& plan, hipStream_t stream);
 int launch_fp8_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                    const afd_ws_layout& L, int32_t n, hipStream_t stream);
+                    const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream);
 
 // Grouped GEMMs for few tokens per expert (afd_gemm_rows.hip), every format; the same results bit
-// for bit. Which GEMMs a call of n tokens launches: rows_plan (afd_rows_rule.h).
+// for bit. Which GEMMs a call launches: its RowsPlan (afd_rows_rule.h).
 // The gate of a GEMM launch: it runs if the router chose its form; few == nullptr: it runs.
 struct RowsGate {
   const int32_t* few;
   __device__ __forceinline__ bool few_skips() const { return few != nullptr && *few == 0; }
   __device__ __forceinline__ bool large_skips() const { return few != nullptr && *few != 0; }
 };
-RowsGate rows_gate(const afd_moe_cfg& cfg, uint8_t* ws, const afd_ws_layout& L, int32_t n);
+RowsGate rows_gate(const RowsPlan& plan, uint8_t* ws, const afd_ws_layout& L);
 // x / xs: the token rows in the activation format (quantized, or bf16 with xs null); with
 // rows_desc != nullptr they are read from that job descriptor when the kernel runs.
 int launch_rows_gate_up(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
                         const afd_ws_layout& L, const void* x, const void* xs,
-                        const afd_job* rows_desc, int32_t n, hipStream_t stream);
+                        const afd_job* rows_desc, const RowsPlan& plan, hipStream_t stream);
 int launch_rows_down(const afd_moe_cfg& cfg, const afd_expert_weights& wt, uint8_t* ws,
-                     const afd_ws_layout& L, int32_t n, hipStream_t stream);
+                     const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream);
 
 // Number of compute units of the current device (cached per device).
 int device_cu_count();

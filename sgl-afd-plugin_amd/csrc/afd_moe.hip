@@ -386,28 +386,28 @@ static int moe_ffn_impl(const afd_moe_cfg* cfg, const afd_expert_weights* weight
       reply = *answer;
       reply.arrive = call_counters(wsb, L) + kArriveWord;
     }
-    st = launch_route_quant(job, !quantized && !a16, *cfg, wsb, L, s,
+    const RowsPlan plan = rows_plan(*cfg, n, job.desc != nullptr);
+    st = launch_route_quant(job, !quantized && !a16, *cfg, wsb, L, plan, s,
                             ev && ev[1] ? static_cast<hipEvent_t>(ev[1]) : nullptr);
     if (st != AFD_OK) return st;
     if ((st = mark(2)) != AFD_OK) return st;
-    const int form = rows_plan(*cfg, n).form;
     const uint16_t* rows = staged_x != nullptr ? staged_x : job.x;
     const uint8_t* aq = quantized ? xq : wsb + L.xq;
     const void* as = quantized ? xs : static_cast<const void*>(wsb + L.xs);
     const afd_job* rows_desc = (a16 ? staged_x == nullptr : quantized) ? job.desc : nullptr;
-    if (form != kRowsLarge)
+    if (plan.form != kRowsLarge)
       st = launch_rows_gate_up(*cfg, *weights, wsb, L, a16 ? static_cast<const void*>(rows) : aq,
-                               a16 ? nullptr : as, rows_desc, n, s);
-    if (form != kRowsFew && st == AFD_OK)
-      st = a16  ? launch_a16_gate_up(*cfg, *weights, wsb, L, rows, rows_desc, n, s)
-           : mx ? launch_mx_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, n, s)
-                : launch_fp8_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, n, s);
+                               a16 ? nullptr : as, rows_desc, plan, s);
+    if (plan.form != kRowsFew && st == AFD_OK)
+      st = a16  ? launch_a16_gate_up(*cfg, *weights, wsb, L, rows, rows_desc, plan, s)
+           : mx ? launch_mx_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, plan, s)
+                : launch_fp8_gate_up(*cfg, *weights, wsb, L, aq, as, rows_desc, plan, s);
     if (st != AFD_OK || (st = mark(3)) != AFD_OK) return st;
-    if (form != kRowsLarge) st = launch_rows_down(*cfg, *weights, wsb, L, n, s);
-    if (form != kRowsFew && st == AFD_OK)
-      st = a16  ? launch_a16_down(*cfg, *weights, wsb, L, n, s)
-           : mx ? launch_mx_down(*cfg, *weights, wsb, L, n, s)
-                : launch_fp8_down(*cfg, *weights, wsb, L, n, s);
+    if (plan.form != kRowsLarge) st = launch_rows_down(*cfg, *weights, wsb, L, plan, s);
+    if (plan.form != kRowsFew && st == AFD_OK)
+      st = a16  ? launch_a16_down(*cfg, *weights, wsb, L, plan, s)
+           : mx ? launch_mx_down(*cfg, *weights, wsb, L, plan, s)
+                : launch_fp8_down(*cfg, *weights, wsb, L, plan, s);
     if (st != AFD_OK || (st = mark(4)) != AFD_OK) return st;
     st = launch_finalize(reinterpret_cast<const uint16_t*>(wsb + L.y),
                          reinterpret_cast<const int32_t*>(wsb + L.pair_pos), job, cfg->topk,

@@ -298,7 +298,7 @@ void route_chunking(int64_t pairs, int* chunks, int* chunk) {
 }
 
 int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, uint8_t* ws,
-                       const afd_ws_layout& L, hipStream_t stream, hipEvent_t mid) {
+                       const afd_ws_layout& L, const RowsPlan& plan, hipStream_t stream, hipEvent_t mid) {
   uint32_t* counters = call_counters(ws, L);
   // grids for job.n tokens (with a descriptor: n_cap; chunks past the job's pairs are empty)
   const int64_t pairs = job.n * cfg.topk;
@@ -318,7 +318,7 @@ int launch_route_quant(const JobIn& job, bool quantize, const afd_moe_cfg& cfg, 
                        reinterpret_cast<int32_t*>(ws + L.sorted_pairs),
                        reinterpret_cast<int32_t*>(ws + L.pair_pos),
                        reinterpret_cast<int32_t*>(ws + L.tile_expert),
-                       reinterpret_cast<int32_t*>(ws + L.num_tiles), pq, rows_plan(cfg, job.n), counters);
+                       reinterpret_cast<int32_t*>(ws + L.num_tiles), pq, plan, counters);
     AFD_CHECK_LAUNCH();
     return AFD_OK;
   };
@@ -355,6 +355,6 @@ extern "C" int afd_route(const int32_t* ids, int32_t n, const afd_moe_cfg* cfg, 
   if ((!ids && n > 0) || !ws) return AFD_ERR_ARG;
   if (ws_bytes < L.total) return AFD_ERR_WORKSPACE;
   const afd::JobIn job{nullptr, nullptr, ids, nullptr, nullptr, n};
-  return afd::launch_route_quant(job, false, *cfg, static_cast<uint8_t*>(ws), L,
+  return afd::launch_route_quant(job, false, *cfg, static_cast<uint8_t*>(ws), L, afd::rows_plan(*cfg, n, false),
                                  static_cast<hipStream_t>(stream), nullptr);
 }

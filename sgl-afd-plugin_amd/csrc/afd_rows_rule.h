@@ -26,7 +26,10 @@ constexpr int kFewRowsPerExpert = 40;
 // the two launches that return at once cost 2 to 5 us (2% at 1200 tokens), which is why this ends a
 // little before 40; and a rank that owns all experts, which would always pay them (64 of 64, 560
 // tokens 209 -> 215 us; 32 of 32 of hidden 2048, 800 tokens 101 -> 105), never launches both for
-// this. Measured up to a quarter, hence the second bound. FP8 experts gain nothing there (32 of 128
+// this. A call whose descriptor holds the token count (a graph of that capacity) does: it may have
+// few tokens (64 of 64, hidden 4096, inter 1024, room for 500: 60 tokens 125 -> 91 us), and so does a
+// call that doesn't say the model's experts: missing the few rows costs more than launching them.
+// Measured up to a quarter, hence the second bound. FP8 experts gain nothing there (32 of 128
 // experts, 512 tokens: 68 -> 74 us) and take the large tiles.
 constexpr int kGatedRowsPerModelExpert = 35, kGatedRowsPerExpert = 140;
 // Groups of 32 rows run three workgroups a CU instead of two, groups of 64 read the weights of an
@@ -63,16 +66,13 @@ struct RowsPlan {
   int32_t group_shift;  // the few-rows GEMMs' groups have 1 << group_shift rows
   int32_t max_pairs;    // kRowsBoth: bounds of rows_few
   int32_t max_groups;
+  int32_t grid_groups;  // the few-rows GEMMs are launched for so many row groups, the most there can be
 };
 
-// The model's experts, as far as the configuration says: at least those up to this rank's last one.
-inline int64_t model_experts(const afd_moe_cfg& cfg) {
-  const int64_t said = cfg.tile_walk >> AFD_NUM_EXPERTS_SHIFT, seen = int64_t(cfg.expert_lo) + cfg.num_local;
-  return said > seen ? said : seen;
-}
-
-inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n) {
+// The plan of a call of n tokens; capacity: of at most n, the job's descriptor holds how many.
+inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n, bool capacity) {
   const int64_t pairs = n * cfg.topk, local = cfg.num_local;
+  const int64_t experts = cfg.tile_walk >> AFD_NUM_EXPERTS_SHIFT;  // the model's; 0: not said
   RowsPlan p;
   const bool narrow = pairs <= kNarrowRowsPerExpert * local;
   p.group_shift = narrow ? 5 : 6;
@@ -82,9 +82,13 @@ inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n) {
     p.form = pairs <= (narrow ? kFewPairsNarrow : kFewPairs) ? kRowsFew : kRowsBoth;
   else
     p.form = cfg.weight_fmt == AFD_W_MXFP4 && pairs <= kGatedRowsPerExpert * local &&
-                     pairs <= kGatedRowsPerModelExpert * model_experts(cfg)
+                     (capacity || experts == 0 || pairs <= kGatedRowsPerModelExpert * experts)
                  ? kRowsBoth
                  : kRowsLarge;
+  // groups of the pairs that the few-rows GEMMs run for: at most one per pair, and one per expert
+  // plus one per full group
+  const int64_t most = pairs < p.max_pairs ? pairs : p.max_pairs, groups = local + (most >> p.group_shift);
+  p.grid_groups = static_cast<int32_t>(most < groups ? most : groups);
   return p;
 }
 

@@ -249,3 +249,27 @@ def test_local_pairs_at_the_line(extra, want, act):
     got = call(n)
     assert int(experts.ws_view("num_tiles", torch.int32, 2, n)[1]) == want
     assert np.array_equal(got, call(n + more)[:n])
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("n,want", [(3, 1), (210, 1), (211, 0), (400, 0)])
+def test_capacity_above_the_line(n, want, act):
+    """A descriptor call with room for 50 pairs per local expert, all experts local: by the tokens it
+    has (40 pairs per expert, and one token more), the few rows or the large tiles."""
+    num_local, k, cap = 42, 8, 400
+    gen = W.generator("cpu", 43)
+    x = W.tokens(cap, 512, gen, "cpu").to(dev())
+    ids, w = W.route_uniform(cap, num_local, k, gen, "cpu")
+    w13, w2 = W.expert_weights(num_local, 512, 256, gen, "cpu")
+    experts = AfdExperts(num_local, k, 0, range(num_local), pack_mxfp4_experts(w13, w2, device=dev()), n_max=cap,
+                         act_format="bf16" if act == "bf16" else None)
+    ids, w = ids.to(torch.int32).to(dev()), w.float().to(dev())
+    experts.workspace().fill_(0xFF)
+    desc, out = new_job_desc(dev()), torch.full((n, 512), float("nan"), dtype=torch.bfloat16, device=dev())
+    set_job(desc, ids=ids[:n], w=w[:n], out=out, x=x[:n])
+    experts.call_job(desc, cap)
+    torch.cuda.synchronize()
+    assert int(experts.ws_view("num_tiles", torch.int32, 2, cap)[1]) == want
+    whole = experts(x, StandardTopKOutput(w, ids))  # its 400 tokens by value: the large tiles
+    torch.cuda.synchronize()
+    assert np.array_equal(bits16(out), bits16(whole)[:n])

@@ -6,6 +6,7 @@ launches them alone only while it is too small for that; a larger one launches b
 router's counts choose."""
 
 import os
+import random
 import shutil
 import subprocess
 
@@ -26,17 +27,23 @@ def rule(tmp_path_factory):
                     "-o", str(exe)], check=True, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
 
     def run(cases):
-        """cases: dicts; returns (form, group rows, the router's choice) of each. ``counts``: rows per expert."""
+        """cases: dicts; returns (form, group rows, the router's choice) of each. ``counts``: rows per
+        expert; ``capacity``: the call's descriptor holds its tokens, n is the most."""
         lines = []
         for c in cases:
             n, k, local = c["n"], c.get("topk", 8), c["local"]
             rows = 32 if n * k <= 16 * local else 64
             counts = c.get("counts", [])
             lines.append(f"{c['fmt']} {c.get('inter', 2048)} {k} {c.get('lo', 0)} {local} {c.get('walk', 0)} {n} "
+                         f"{c.get('capacity', 0)} "
                          f"{sum(counts)} {sum(-(-v // rows) for v in counts)} {sum(v > 0 for v in counts)}")
         res = subprocess.run([str(exe)], input="\n".join(lines) + "\n", stdout=subprocess.PIPE, text=True, timeout=60,
                              check=True)
-        return [tuple(int(v) for v in line.split()) for line in res.stdout.splitlines()]
+        got = [tuple(int(v) for v in line.split()) for line in res.stdout.splitlines()]
+        for c, (form, rows, choice, grid_groups) in zip(cases, got):  # the launch covers whatever runs
+            groups = sum(-(-v // rows) for v in c.get("counts", []))
+            assert form == LARGE or form == BOTH and not choice or groups <= grid_groups, c
+        return [g[:3] for g in got]
 
     return run
 
@@ -48,7 +55,7 @@ def test_form_and_group_rows_at_the_lines(rule, fmt):
         (dict(local=64, n=128), (FEW, 32)),  # 16 pairs per expert
         (dict(local=64, n=129), (FEW, 64)),
         (dict(local=64, n=320), (FEW, 64)),  # 40 pairs per expert, 2560 pairs
-        (dict(local=64, n=321, walk=256 << 8), (BOTH if fmt == MXFP4 else LARGE, 64)),
+        (dict(local=64, n=321), (BOTH if fmt == MXFP4 else LARGE, 64)),
         (dict(local=65, n=2560, topk=1), (FEW, 64)),
         (dict(local=65, n=2561, topk=1), (BOTH, 64)),
         (dict(local=256, n=256), (FEW, 32)),  # 2048 pairs
@@ -95,12 +102,11 @@ def test_few_rows_run_alone_only_in_small_calls(rule, fmt, local, inter):
 
 
 @pytest.mark.parametrize("lo,said,last", [
-    (0, 0, 320),  # 64 experts, as far as the configuration says: all local
     (0, 64, 320),  # all local
     (0, 65, 320), (0, 80, 350),  # the few-rows line itself; 35 pairs per expert of the model
-    (0, 128, 560), (64, 0, 560), (64, 128, 560),  # half
-    (0, 256, 1120), (192, 0, 1120), (64, 256, 1120),  # a quarter
-    (0, 512, 1120), (448, 0, 1120),  # an eighth: measured up to a quarter
+    (0, 128, 560), (64, 128, 560),  # half
+    (0, 256, 1120), (192, 256, 1120), (0, 0, 1120), (64, 0, 1120),  # a quarter; not said
+    (0, 512, 1120),  # an eighth: measured up to a quarter
 ])
 def test_both_forms_are_launched_only_near_the_line(rule, lo, said, last):
     """An MXFP4 rank launches both forms for the count of local pairs only where its share of the
@@ -110,3 +116,29 @@ def test_both_forms_are_launched_only_near_the_line(rule, lo, said, last):
     assert [form for form, _, _ in got] == [FEW if n <= 320 else BOTH if n <= last else LARGE for n in sizes]
     got = rule([dict(fmt=FP8_BLOCK, local=64, lo=lo, n=n, walk=said << 8 | n % 2) for n in sizes])
     assert [form for form, _, _ in got] == [FEW if n <= 320 else LARGE for n in sizes]
+    # a capacity: the job may have few tokens, so the count decides up to 140 pairs per expert
+    got = rule([dict(fmt=MXFP4, local=64, lo=lo, n=n, walk=said << 8 | n % 2, capacity=1) for n in sizes])
+    assert [form for form, _, _ in got] == [FEW if n <= 320 else BOTH if n <= 1120 else LARGE for n in sizes]
+
+
+def test_the_launch_covers_every_routing(rule):
+    """Random loads, even to concentrated: the few-rows grid has a group for each that can be."""
+    rng = random.Random(3)
+    cases = []
+    for _ in range(4000):
+        local = rng.choice([1, 2, 5, 64, 65, 128, 256])
+        k = rng.randint(1, 8)
+        n = rng.randint(1, max(1, 45 * local // k))
+        hot = rng.randint(1, local)
+        counts = [0] * local
+        left = rng.choice([n * k, rng.randint(0, n * k)])
+        for e in range(hot):
+            counts[e] = left // hot + (e < left % hot)
+        for _ in range(hot):
+            a, b = rng.randrange(hot), rng.randrange(hot)
+            moved = rng.randint(0, counts[a])
+            counts[a] -= moved
+            counts[b] += moved
+        cases.append(dict(fmt=rng.choice([MXFP4, FP8_BLOCK]), local=local, topk=k, n=n, counts=counts,
+                          inter=rng.choice([128, 1024, 2048, 16384]), walk=4 * local << 8))
+    rule(cases)
