@@ -78,8 +78,11 @@ inline RowsPlan rows_plan(const afd_moe_cfg& cfg, int64_t n, bool capacity) {
   p.group_shift = narrow ? 5 : 6;
   p.max_pairs = static_cast<int32_t>(kFewRowsPerExpert * local);
   p.max_groups = kRowsRounds * (narrow ? 3 : 2) * kRowsCus / (2 * cfg.inter / 256);
+  // The counts say large tiles only if 2 groups > 3 active; with groups <= active + pairs / rows that
+  // takes more than max_groups <= groups < 3 pairs / rows.
+  const bool always_few = 3 * pairs <= int64_t(p.max_groups) << p.group_shift;
   if (pairs <= kFewRowsPerExpert * local)
-    p.form = pairs <= (narrow ? kFewPairsNarrow : kFewPairs) ? kRowsFew : kRowsBoth;
+    p.form = always_few || pairs <= (narrow ? kFewPairsNarrow : kFewPairs) ? kRowsFew : kRowsBoth;
   else
     p.form = cfg.weight_fmt == AFD_W_MXFP4 && pairs <= kGatedRowsPerExpert * local &&
                      (capacity || experts == 0 || pairs <= kGatedRowsPerModelExpert * experts)

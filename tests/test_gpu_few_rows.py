@@ -135,7 +135,8 @@ def test_concentrated_rows_match_large_tiles(num_local, counts, fmt, act):
     assert np.array_equal(few, call(n + more)[:n])
 
 
-# Above 2560 pairs (2048 in groups of 32 rows) a call launches both forms and the router writes its
+# Above 2560 pairs (2048 in groups of 32 rows), if some routing could call for the large tiles, a call
+# launches both forms and the router writes its
 # choice: few rows if gate_up's row groups make at most two rounds of workgroups (1024 / image columns
 # groups of 64 rows, 1536 / columns of 32), or there are at most 3/2 groups per expert with rows.
 def spread(experts, rows, last):
@@ -155,7 +156,9 @@ EDGES = [
     (256, 256, 2048, spread(31, 65, 97), 0),  # 97
     (256, 256, 2048, spread(80, 33, 0) + spread(80, 1, 0), 1),  # 240 on 160: 3/2
     (256, 256, 2048, spread(81, 33, 0) + spread(79, 1, 0), 0),  # 241 on 160
-    (256, 256, 128, [0] * 255 + [4000], 1),  # one column; all rows on the last expert
+    # one column: no routing makes two rounds, so the few rows run alone (no choice written); all rows
+    # on the last expert
+    (256, 256, 128, [0] * 255 + [4000], -1),
 ]
 
 

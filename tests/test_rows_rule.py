@@ -18,6 +18,10 @@ LARGE, FEW, BOTH = 0, 1, 2
 MXFP4, FP8_BLOCK = 1, 2
 
 
+def n_pairs(case):
+    return case["n"] * case.get("topk", 8)
+
+
 @pytest.fixture(scope="module")
 def rule(tmp_path_factory):
     if not os.path.exists(HIPCC):
@@ -43,6 +47,8 @@ def rule(tmp_path_factory):
         for c, (form, rows, choice, grid_groups) in zip(cases, got):  # the launch covers whatever runs
             groups = sum(-(-v // rows) for v in c.get("counts", []))
             assert form == LARGE or form == BOTH and not choice or groups <= grid_groups, c
+            # alone above 2560 pairs only where no routing makes the counts say otherwise
+            assert form != FEW or n_pairs(c) <= 2560 or choice, c
         return [g[:3] for g in got]
 
     return run
@@ -87,7 +93,7 @@ def test_concentrated_routing_takes_the_large_tiles(rule, fmt):
     assert [choice for _, _, choice in got] == [0] * len(large) + [1] * len(few)
 
 
-@pytest.mark.parametrize("local,inter", [(64, 2048), (65, 1536), (128, 2048), (256, 1024), (256, 2048)])
+@pytest.mark.parametrize("local,inter", [(64, 2048), (65, 1536), (128, 2048), (256, 512), (256, 1024), (256, 2048)])
 @pytest.mark.parametrize("fmt", [MXFP4, FP8_BLOCK])
 def test_few_rows_run_alone_only_in_small_calls(rule, fmt, local, inter):
     sizes = list(range(1, 6 * local))
@@ -97,7 +103,9 @@ def test_few_rows_run_alone_only_in_small_calls(rule, fmt, local, inter):
         if pairs > 40 * local:
             assert form == (BOTH if fmt == MXFP4 and pairs <= 140 * local else LARGE), n
         else:
-            assert form == (FEW if pairs <= (2048 if rows == 32 else 2560) else BOTH), n
+            rounds = (1536 if rows == 32 else 1024) // (inter // 128)  # row groups of two rounds
+            alone = pairs <= (2048 if rows == 32 else 2560) or 3 * pairs <= rounds * rows
+            assert form == (FEW if alone else BOTH), n
             assert rows == (32 if pairs <= 16 * local else 64), n
 
 
