@@ -43,6 +43,7 @@
 #include <type_traits>
 
 #include "afd_common.h"
+#include "afd_gemm_dev.h"
 #include "afd_internal.h"
 
 namespace afd {
@@ -53,8 +54,6 @@ enum { kGateUp = 0, kDown = 1, kGateUpParam = 2 };
 enum { kWMx = 0, kWFp8 = 1 };  // weight format of the kernel
 
 constexpr int kA16WalkRows = 4;
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 struct A16GemmArgs {
   const uint8_t* a_img;         // down: bf16 A images [row tiles][K / stage K]
@@ -131,36 +130,6 @@ struct A16Tile {
   static_assert(kLds <= 160 * 1024, "LDS of one CU");
   static_assert(kStages * (kPiecesMin + 1) < 64, "vmcnt is a 6-bit counter");
 };
-
-// the 8 e2m1 codes of dword d (element 2i in the low nibble of byte i) times 2^(code - 127),
-// as the 8 bf16 of an MFMA operand (element i in half i % 2 of dword i / 2). The instruction
-// takes the scale's exponent field as the UE8M0 code, so `scale` is the code shifted into it.
-__device__ __forceinline__ v8bf expand_fp4(uint32_t d, float scale) {
-  v4i r;
-  r[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 0));
-  r[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 1));
-  r[2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 2));
-  r[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 3));
-  return __builtin_bit_cast(v8bf, r);
-}
-
-// the 8 e4m3 codes of dwords d0, d1 (element i in byte i % 4 of dword i / 4) as the 8 bf16 of
-// an MFMA operand, exactly (scale 2^0)
-__device__ __forceinline__ v8bf expand_fp8(uint32_t d0, uint32_t d1) {
-  v4i r;
-  r[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d0, 1.0f, false));
-  r[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d0, 1.0f, true));
-  r[2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d1, 1.0f, false));
-  r[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d1, 1.0f, true));
-  return __builtin_bit_cast(v8bf, r);
-}
-
-// A uniform read of data the kernel never writes (the FP8 block scales), through the scalar
-// cache: read through a generic pointer the compiler has to assume a store of the kernel may
-// alias it and issues a vector load, whose wait then drains the copies in flight.
-__device__ __forceinline__ float load_uniform(const float* p) {
-  return *(const __attribute__((address_space(4))) float*)p;
-}
 
 template <int WF, int MODE, int WN>
 __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A16GemmArgs p) {
@@ -504,21 +473,6 @@ __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A
     // 128 wn + 32 j + 8 (q / 4) + 4 (lane / 32) + q % 4. Lane half lk holds columns
     // 8 q4 + 4 lk .. + 3 of each 32-column tile; one v_permlane32_swap per pair of bf16 pairs
     // gives lane half lk the whole 16-byte chunks 2 pr + lk (pr = 0, 1), in column order.
-    auto chunks_of = [&](const float (&h)[16], v4i (&chunk)[2]) {
-      uint32_t hb[4][2];
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        hb[q4][0] = pk_bf16(h[4 * q4], h[4 * q4 + 1]);
-        hb[q4][1] = pk_bf16(h[4 * q4 + 2], h[4 * q4 + 3]);
-      }
-#pragma unroll
-      for (int pr = 0; pr < 2; ++pr) {
-        const auto d0 = __builtin_amdgcn_permlane32_swap(hb[2 * pr][0], hb[2 * pr + 1][0], false, false);
-        const auto d1 = __builtin_amdgcn_permlane32_swap(hb[2 * pr][1], hb[2 * pr + 1][1], false, false);
-        chunk[pr] = v4i{static_cast<int>(d0[0]), static_cast<int>(d1[0]), static_cast<int>(d0[1]),
-                        static_cast<int>(d1[1])};
-      }
-    };
     if constexpr (MODE != kDown) {
       // Column tiles j = 2 jj and 2 jj + 1 are the gate and up halves of one 64-row group of
       // interleaved W13: the same 32 intermediate columns n0 / 2 + 64 wn + 32 jj + [0, 32).
@@ -537,7 +491,7 @@ __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A
             for (int q = 0; q < 16; ++q)
               h[q] = fn(acc[i2][2 * jj][q] * s_run[0], acc[i2][2 * jj + 1][q] * s_run[1]);
             v4i chunk[2];
-            chunks_of(h, chunk);
+            bf16_chunks(h, chunk);
             const int col0 = n0 / 2 + 64 * wn + 32 * jj;  // multiple of 32
             uint8_t* img = p.h_img + (int64_t(mt) * kt_down + col0 / kStageK) * T::kLdsA;
 #pragma unroll
@@ -573,7 +527,7 @@ __global__ __launch_bounds__((A16Tile<WF, WN>::kThreads)) void a16_gemm_kernel(A
 #pragma unroll
           for (int q = 0; q < 16; ++q) h[q] = acc[i2][j][q] * s_run[0];
           v4i chunk[2];
-          chunks_of(h, chunk);
+          bf16_chunks(h, chunk);
 #pragma unroll
           for (int pr = 0; pr < 2; ++pr)
             *reinterpret_cast<v4i*>(lds + y_chunk(row, (wn * 128 + j * 32) / 8 + 2 * pr + lk)) = chunk[pr];

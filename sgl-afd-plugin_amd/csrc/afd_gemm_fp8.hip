@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "afd_common.h"
+#include "afd_gemm_dev.h"
 #include "afd_internal.h"
 
 namespace afd {
@@ -119,12 +120,6 @@ struct Tile {
   static constexpr int lds_bytes() { return MODE == 1 ? kDownLds : kGateUpLds; }
   static_assert(4 * (kPiecesMin + 1) < 64 && kQP + 2 * (kGAQ + kQP) + 1 < 64, "vmcnt is a 6-bit counter");
 };
-
-// A uniform read of data the kernel never writes (the weight block scales), through the
-// scalar cache: a vector load's wait would drain the copies in flight.
-__device__ __forceinline__ float load_uniform(const float* p) {
-  return *(const __attribute__((address_space(4))) float*)p;
-}
 
 template <int MODE>
 __global__ __launch_bounds__(Tile::kThreads) void fp8_gemm_kernel(Fp8GemmArgs p) {
@@ -588,15 +583,7 @@ __global__ __launch_bounds__(Tile::kThreads) void fp8_gemm_kernel(Fp8GemmArgs p)
             for (int q4 = 0; q4 < 4; ++q4)
               d[q4] = pk4_e4m3_near(div_by(h[i2][jj][4 * q4], sc, rsc), div_by(h[i2][jj][4 * q4 + 1], sc, rsc),
                                div_by(h[i2][jj][4 * q4 + 2], sc, rsc), div_by(h[i2][jj][4 * q4 + 3], sc, rsc));
-            // lane half 0 takes columns 0-15 (its d0, d1 and the partner's), half 1 columns
-            // 16-31 (the partner's d2, d3 and its own)
-            const uint32_t p0 = swap_halves(d[2], d[0], lk);
-            const uint32_t p1 = swap_halves(d[3], d[1], lk);
-            v4i chunk;
-            chunk[0] = static_cast<int>(lk ? p0 : d[0]);
-            chunk[1] = static_cast<int>(lk ? d[2] : p0);
-            chunk[2] = static_cast<int>(lk ? p1 : d[1]);
-            chunk[3] = static_cast<int>(lk ? d[3] : p1);
+            const v4i chunk = e4m3_chunk(d, lk);
             const int col0 = n0 / 2 + 64 * wn + 32 * jj;  // multiple of 32
             uint8_t* img = p.hq + (int64_t(mt) * (inter / kF8K) + col0 / kF8K) * kImgF8B;
             *reinterpret_cast<v4i*>(img + img_b_off(row, (col0 % kF8K) / 16 + lk)) = chunk;

@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "afd_common.h"
+#include "afd_gemm_dev.h"
 #include "afd_internal.h"
 
 namespace afd {
@@ -91,14 +92,6 @@ struct MxTile {
   static_assert(kLds <= 160 * 1024, "LDS of one CU");
   static_assert(2 * kPieces < 64, "vmcnt is a 6-bit counter");
 };
-
-// The scaled MFMA with a 4-dword (e2m1) B operand. The clang builtin takes 8 dwords for every
-// operand format; the intrinsic's B operand type follows the format, and e2m1 needs only 4.
-// The kernels pass the e2m1 weights as the first operand and the e4m3 activations as the
-// second (D = W X^T), so a lane's accumulators belong to one activation row.
-extern "C" __device__ v16f mfma_scale_f4_f8(v4i a, v8i b, v16f c, int cbsz, int blgp,
-                                            int opsel_a, int scale_a, int opsel_b, int scale_b)
-    __asm("llvm.amdgcn.mfma.scale.f32.32x32x64.f8f6f4.v4i32.v8i32");
 
 // kCont false: each tile fills the ring, runs its K loop, drains the ring and runs its
 // epilogue. kCont (gate_up with at least 3 K stages, static walk): the copy ring runs on across
@@ -357,15 +350,7 @@ __global__ __launch_bounds__(MxTile<WN>::kThreads) void mx_gemm_kernel(MxGemmArg
           for (int q4 = 0; q4 < 4; ++q4)
             d[q4] = pk4_e4m3(h[4 * q4] * inv, h[4 * q4 + 1] * inv, h[4 * q4 + 2] * inv,
                              h[4 * q4 + 3] * inv);
-          // lane half 0 takes columns 0-15 (its d0, d1 and the partner's), half 1 columns
-          // 16-31 (the partner's d2, d3 and its own)
-          const uint32_t p0 = swap_halves(d[2], d[0], lk);
-          const uint32_t p1 = swap_halves(d[3], d[1], lk);
-          v4i chunk;
-          chunk[0] = static_cast<int>(lk ? p0 : d[0]);
-          chunk[1] = static_cast<int>(lk ? d[2] : p0);
-          chunk[2] = static_cast<int>(lk ? p1 : d[1]);
-          chunk[3] = static_cast<int>(lk ? d[3] : p1);
+          const v4i chunk = e4m3_chunk(d, lk);
           const int row = wm * 64 + i * 32 + lr;
           const int hblk = wn * 2 + jj;  // MX block among the tile's kBN / 64
           uint8_t* img = p.h_img + (int64_t(mt) * kt_down + n0 / kImgBRows + hblk / 4) * kImgA;

@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "afd_common.h"
+#include "afd_gemm_dev.h"
 #include "afd_internal.h"
 
 namespace afd {
@@ -38,8 +39,6 @@ namespace {
 enum { kGateUp = 0, kDown = 1, kGateUpParam = 2 };
 // weight x activation formats: MXFP4 x MXFP8, FP8 block x FP8 1x128, MXFP4 x bf16, FP8 x bf16
 enum { kMx8 = 0, kF8 = 1, kMx16 = 2, kF16 = 3 };
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 struct RowsArgs {
   const uint8_t* a;          // gate_up: token rows [n][K] (e4m3 or bf16); down: the h images
@@ -73,30 +72,6 @@ struct Fmt {
   static constexpr int kALoads = kABlock / 4096;      // 16-byte loads of a lane per block (4 wavefronts)
 };
 
-// The scaled MFMA with a 4-dword (e2m1) first operand (see afd_gemm_mx.hip).
-extern "C" __device__ v16f mfma_scale_rows_f4_f8(v4i a, v8i b, v16f c, int cbsz, int blgp, int opsel_a,
-                                                 int scale_a, int opsel_b, int scale_b)
-    __asm("llvm.amdgcn.mfma.scale.f32.32x32x64.f8f6f4.v4i32.v8i32");
-
-__device__ __forceinline__ v8bf expand_fp4(uint32_t d, float scale) {
-  v4i r;
-  r[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 0));
-  r[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 1));
-  r[2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 2));
-  r[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(d, scale, 3));
-  return __builtin_bit_cast(v8bf, r);
-}
-__device__ __forceinline__ v8bf expand_fp8(uint32_t d0, uint32_t d1) {
-  v4i r;
-  r[0] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d0, 1.0f, false));
-  r[1] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d0, 1.0f, true));
-  r[2] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d1, 1.0f, false));
-  r[3] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d1, 1.0f, true));
-  return __builtin_bit_cast(v8bf, r);
-}
-__device__ __forceinline__ float load_uniform(const float* p) {
-  return *(const __attribute__((address_space(4))) float*)p;
-}
 // Global-memory pointers by type: read through a generic one (a row pointer may come from the job
 // descriptor) the compiler would issue flat loads, whose waits also count LDS operations.
 typedef const __attribute__((address_space(1))) uint8_t* GPtr;
@@ -366,7 +341,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
             const v8i fa = join(a_chunk(i, 2 * ks), a_chunk(i, 2 * ks + 1));
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-              acc[i][j] = mfma_scale_rows_f4_f8(w4[j][ks], fa, acc[i][j], 4 /*A e2m1*/, 0 /*B e4m3*/, ks,
+              acc[i][j] = mfma_scale_f4_f8(w4[j][ks], fa, acc[i][j], 4 /*A e2m1*/, 0 /*B e4m3*/, ks,
                                                 static_cast<int>(sb[j]), ks, static_cast<int>(f.sa[i]));
           }
         });
@@ -478,33 +453,6 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
     bool real[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) real[i] = r0 + 32 * i + lr < live;
-    // lane half lk's whole 16-byte chunks 2 pr + lk of the 32 bf16 columns
-    auto bf16_chunks = [&](const float (&h)[16], v4i (&chunk)[2]) {
-      uint32_t hb[4][2];
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        hb[q4][0] = pk_bf16(h[4 * q4], h[4 * q4 + 1]);
-        hb[q4][1] = pk_bf16(h[4 * q4 + 2], h[4 * q4 + 3]);
-      }
-#pragma unroll
-      for (int pr = 0; pr < 2; ++pr) {
-        const auto d0 = __builtin_amdgcn_permlane32_swap(hb[2 * pr][0], hb[2 * pr + 1][0], false, false);
-        const auto d1 = __builtin_amdgcn_permlane32_swap(hb[2 * pr][1], hb[2 * pr + 1][1], false, false);
-        chunk[pr] = v4i{static_cast<int>(d0[0]), static_cast<int>(d1[0]), static_cast<int>(d0[1]),
-                        static_cast<int>(d1[1])};
-      }
-    };
-    // the 16 e4m3 codes of lane half lk: columns 16 lk .. 16 lk + 15 of the 32
-    auto fp8_chunk = [&](const uint32_t (&d)[4]) {
-      const uint32_t p0 = swap_halves(d[2], d[0], lk);
-      const uint32_t p1 = swap_halves(d[3], d[1], lk);
-      v4i chunk;
-      chunk[0] = static_cast<int>(lk ? p0 : d[0]);
-      chunk[1] = static_cast<int>(lk ? d[2] : p0);
-      chunk[2] = static_cast<int>(lk ? p1 : d[1]);
-      chunk[3] = static_cast<int>(lk ? d[3] : p1);
-      return chunk;
-    };
     if constexpr (kGU) {
       auto store_h = [&](auto fn) __attribute__((always_inline)) {
         float h[NB][16], m[NB];
@@ -542,7 +490,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
             for (int q4 = 0; q4 < 4; ++q4)
               d[q4] = pk4_e4m3(h[i][4 * q4] * inv, h[i][4 * q4 + 1] * inv, h[i][4 * q4 + 2] * inv,
                                h[i][4 * q4 + 3] * inv);
-            const v4i chunk = fp8_chunk(d);
+            const v4i chunk = e4m3_chunk(d, lk);
             // MX block w of the 4 in K stage nt of the down GEMM
             uint8_t* img = p.hq + (int64_t(mt) * ntn + nt) * kImgA;
             if (real[i]) {
@@ -557,7 +505,7 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 2) void rows_gemm_kernel(RowsArgs
             for (int q4 = 0; q4 < 4; ++q4)
               d[q4] = pk4_e4m3_near(div_by(h[i][4 * q4], sc, rsc), div_by(h[i][4 * q4 + 1], sc, rsc),
                                     div_by(h[i][4 * q4 + 2], sc, rsc), div_by(h[i][4 * q4 + 3], sc, rsc));
-            const v4i chunk = fp8_chunk(d);
+            const v4i chunk = e4m3_chunk(d, lk);
             uint8_t* img = p.hq + (int64_t(mt) * ntn * 2 + 2 * nt + (w >> 1)) * kImgF8B;
             if (real[i]) {
               *reinterpret_cast<v4i*>(img + img_b_off(r, 2 * (w & 1) + lk)) = chunk;
