@@ -8,8 +8,8 @@
 // Split: a workgroup of 4 wavefronts owns a row group (at most 32 R = 32 or 64 rows of one
 // expert) x the 256 weight rows of one image column; wavefront w streams its 64 rows (gate_up: 32 gate and the
 // matching 32 up rows; 4 KiB of each image) over the whole K from HBM into registers, several K
-// stages of 128 ahead, so 256-column items fill the chip and 2 or 3 workgroups a CU keep 70-150 KB
-// of weights in flight. A stage passes through LDS on its way to the matrix instructions: the
+// stages of 128 ahead (depth()), so 256-column items fill the chip and 2 or 3 workgroups a CU keep
+// 104-209 KB of weights in flight. A stage passes through LDS on its way to the matrix instructions: the
 // weights through the wavefront's own area, which lets the loads be contiguous kilobytes (read in
 // fragment order, half a line a load, non-temporal loads reach 5.3 TB/s here and default ones
 // 6.1; contiguous non-temporal ones 7.0), the activations through a block the four wavefronts fill

@@ -379,8 +379,9 @@ static int moe_ffn_impl(const afd_moe_cfg* cfg, const afd_expert_weights* weight
   if (n > 0) {
     uint8_t* wsb = static_cast<uint8_t*>(ws);
     const bool mx = cfg->weight_fmt == AFD_W_MXFP4;
-    // routing and the activation quantization (one launch beside the expert histogram), then
-    // the pair scatter; stage mark 1 falls between the two launches
+    // routing and the activation quantization: one launch, which stage mark 1 follows, or above
+    // 4096 pairs two (quantization beside the expert histogram, then the pair scatter) with mark 1
+    // between them
     Reply reply = {};
     if (answer != nullptr) {
       reply = *answer;

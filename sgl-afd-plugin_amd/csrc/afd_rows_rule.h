@@ -15,7 +15,9 @@ namespace afd {
 // catch up (large tiles -> few rows): 64 FP8 experts, all local, hidden 4096, inter 1536, top-8: at
 // 37 pairs per expert 278 -> 234 us (uniform routing) and 328 -> 283 (Zipf 1.2), at 64 285 -> 339
 // and 343 -> 346; MXFP4 experts, hidden 4096, inter 2048: at 32 200 -> 189 us (uniform) and
-// 236 -> 222 (Zipf 1.2), at 48 210 -> 225 and 245 -> 259, with bf16 activations at 35 366 -> 270.
+// 236 -> 222 (Zipf 1.2), at 48 210 -> 225 and 245 -> 259. With bf16 activations they catch up a
+// little later: MXFP4 at 40 250 -> 235 and 369 -> 253, at 65 300 -> 319 and 386 -> 320; FP8 at 40
+// 275 -> 249 and 322 -> 276, at 65 318 -> 347 and 347 -> 344; and so they do in narrow layers.
 constexpr int kFewRowsPerExpert = 40;
 // A call knows its own pairs, not how many of them are local: with at most 40 pairs per local
 // expert if all were, the few-rows GEMMs run. An MXFP4 rank that owns a quarter of a model's experts
