@@ -780,7 +780,8 @@ def main():
         "six stage events; the timed steps call afd_moe_ffn with no events, and roofline.kernel_ms "
         "comes from a second pass with events around gate_up only. hist_quant: the expert "
         "histogram and the activation quantization in one launch; scatter: the router's scan and "
-        "pair scatter",
+        "pair scatter (a call of at most 4096 pairs does all of it in one launch, which hist_quant "
+        "holds, and scatter is the spacing of two events with no kernel between them)",
         "roofline": {
             "kernel": f"grouped gate_up GEMM + SwiGLU ({kernel})",
             "bound": "mfma",
