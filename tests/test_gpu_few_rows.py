@@ -276,3 +276,28 @@ def test_capacity_above_the_line(n, want, act):
     whole = experts(x, StandardTopKOutput(w, ids))  # its 400 tokens by value: the large tiles
     torch.cuda.synchronize()
     assert np.array_equal(bits16(out), bits16(whole)[:n])
+
+
+@pytest.mark.parametrize("act", ["fp8", "bf16"])
+@pytest.mark.parametrize("fmt", ["mxfp4", "fp8_block"])
+def test_one_local_expert(fmt, act):
+    """One expert: 1 to 40 of its rows, from one group of 32 rows to one of 64, and none."""
+    gen = W.generator("cpu", 47)
+    x = W.tokens(300, 512, gen, "cpu").to(dev())
+    w13, w2 = W.expert_weights(1, 512, 256, gen, "cpu")
+    pack = pack_mxfp4_experts if fmt == "mxfp4" else pack_fp8_block_experts
+    experts = AfdExperts(9, 1, 0, range(4, 5), pack(w13, w2, device=dev()), n_max=300,
+                         act_format="bf16" if act == "bf16" else None)
+    w = (torch.rand(300, 1, generator=gen) + 0.25).to(dev())
+    ids = torch.full((300, 1), 4, dtype=torch.int32, device=dev())
+
+    def call(m, which):
+        experts.workspace().fill_(0xFF)
+        out = experts(x[:m], StandardTopKOutput(w[:m], which[:m]))
+        torch.cuda.synchronize()
+        return bits16(out)
+
+    whole = call(300, ids)  # large tiles
+    for n in (1, 16, 17, 32, 33, 40):
+        assert np.array_equal(call(n, ids), whole[:n]), n
+    assert not call(40, ids + 1).any()
